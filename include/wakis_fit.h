@@ -173,17 +173,20 @@ typedef struct wf_step_args {
   /* Fused path: 1 = advance two steps per launch (temporal blocking) where
    * the two-step kernel applies: FP32 or FP64 storage (not compute_f64),
    * material codes with zero_masked and no escape code, the beam line fed
-   * from beam_table (with or without conduction), Nx <= 256 and a multiple of
-   * the cells per lane (4 FP32, 2 FP64), row segments (variant 0, full_rows
-   * <= 0, cells_per_lane 0 or the cells per lane), no box, no trajectory, no
-   * monitor; otherwise one step per launch. An odd step count ends with one
-   * single step. Results are identical to one step per launch. 0 = one step
-   * per launch; 4 or 8: two steps per launch with that many rows per
-   * workgroup (FP64 always 2 rows, two waves per row); 1 = 8 rows (FP64 2) on
-   * grids of 2^20 cells or more, FP64 also with Nx >= 224 (otherwise one step
-   * per launch is as fast or faster). */
+   * from beam_table (with or without conduction), row segments (variant 0,
+   * full_rows <= 0, cells_per_lane 0 or 16 bytes of cells), every 3N array
+   * within 4 GiB, no box, no trajectory, no monitor; otherwise one step per
+   * launch. Results are identical to one step per launch. 0 = one step per
+   * launch; 4 or 8: two steps per launch with at most that many rows per
+   * workgroup.
+   * E2 and H2 hold the fields one step back after a call, except (fields two
+   * steps back) after an even count with Nx <= 256 a multiple of 4 (FP64: 2)
+   * and two_step 4 or 8, or 1 on grids of 2^20 cells or more (FP64 also
+   * Nx >= 224): such a call takes all its steps in pairs, every other one its
+   * last step or two singly. */
   int32_t two_step;
-  int32_t two_step_used;  /* out: 1 if the call ran two steps per launch            */
+  int32_t two_step_used;  /* out: two steps per launch, 1: to the call's end (but an
+                           * odd step), 2: up to its single last steps            */
 } wf_step_args;
 
 int wf_version(void);

@@ -121,8 +121,11 @@ WF_HIDDEN int noalloc_scratch(long long **out);
 
 // The fused single-pass step (path 1) for FP32 and FP64 storage.
 WF_HIDDEN int step_fused_f32(wf_handle *h, wf_step_args *a, hipStream_t st);
-// two steps per launch (lib_fused_t2.hip): 1 if this call qualifies
+// two steps per launch (lib_fused_t2.hip): 0 if this call does not qualify, 1 if
+// it may end with a pair of steps, 2 if it has to end with a single step
 WF_HIDDEN int fused_t2_applies(const wf_handle *h, const wf_step_args *a);
-WF_HIDDEN int step_fused_t2_f32(wf_handle *h, wf_step_args *a, hipStream_t st);
-WF_HIDDEN int step_fused_t2_f64(wf_handle *h, wf_step_args *a, hipStream_t st);
+WF_HIDDEN int step_fused_t2_f32(wf_handle *h, wf_step_args *a, hipStream_t st,
+                                bool end_paired);
+WF_HIDDEN int step_fused_t2_f64(wf_handle *h, wf_step_args *a, hipStream_t st,
+                                bool end_paired);
 WF_HIDDEN int step_fused_f64(wf_handle *h, wf_step_args *a, hipStream_t st);

@@ -2,80 +2,189 @@
 // material codes, masks folded into the coefficients (zero_masked), the beam
 // line fed from the beam table, with or without conduction (COND: J = sigma E
 // everywhere, recomputed from E as in k_fused4 and stored by the last launch
-// of a call), rows of Nx <= 256 cells: one wave per row with FP32 (V = 4
-// cells per lane), two waves per row with FP64 (V = 2).
+// of a call).
 //
-// A workgroup owns TY rows j0 .. j0+TY-1 and a chunk of z-planes and marches
-// up in z like k_fused4, but carries two time levels, the second one plane
-// behind the first: at plane k it computes step n+1 (level 1: H1(k), E1(k))
-// and step n+2 at plane k-1 (level 2: H2(k-1), E2(k-1)), and stores only
-// level 2. Level 2 on the own rows needs level-1 values on rows j0-1 .. j0+TY
-// (E1) and j0-2 .. j0+TY (H1), so the workgroup has TY + 4 rows of waves,
-// row w = j0-2+w (the last one only stages E0 of row j0+TY+1); halo values are
-// recomputed, never exchanged. Every value is formed by the same expression
-// as in k_fused4 (h_row, e_sum, the coefficient recomputation from the
-// codes), so both levels are bit-identical to two single steps.
+// A workgroup owns T rows of OW cells (both chosen by the host for the grid)
+// and a chunk of z-planes and marches up in z like k_fused4, but carries two
+// time levels, the second one plane behind the first: at plane k it computes
+// step n+1 (level 1: H1(k), E1(k)) and step n+2 at plane k-1 (level 2: H2(k-1),
+// E2(k-1)), and stores only level 2. Level 2 on the own rows needs level-1
+// values on rows j0-1 .. j0+T (E1) and j0-2 .. j0+T (H1), so the workgroup
+// holds T + 4 rows, row r = j0-2+r (the last one only stages E0 of row
+// j0+T+1); along x it holds one lane (V cells) more on each side of the own
+// cells, unless one tile spans the row. Halo values are recomputed, never
+// exchanged. Every value is formed by the same expression as in k_fused4
+// (h_row, e_sum, the coefficient recomputation from the codes), so both levels
+// are bit-identical to two single steps.
+//
+// Thread t holds the V cells of lane t % Q of row t / Q, so rows of any length
+// fill the waves; a lane that the row end cuts loads and stores its cells one
+// at a time, the others with 16-byte accesses at the alignment the row has.
+// A staged row is Q lanes, the first of them without cells where a tile starts
+// at the row's first cell (its zeros are the cells before this row and after
+// the previous one), and lies in LDS in thread order: 64 lanes then take 64
+// consecutive words (a gap between the rows of a wave cost a second pass of
+// every access). Rows of exactly whole waves keep the gap instead of the lane.
 //
 // Per plane, with one barrier after each phase:
-//   P1 H1(k) on waves 0..TY+2; stage H1(k)
-//   P2 E1(k) on waves 1..TY+2; H2(k-1) on waves 1..TY+1 (reads E1(k-1)
-//      staged in the previous P3); stage H2(k-1)
+//   P1 H1(k) on rows 0..T+2; stage H1(k)
+//   P2 E1(k) on rows 1..T+2; H2(k-1) on rows 1..T+1 (reads E1(k-1) staged in
+//      the previous P3); stage H2(k-1)
 //   P3 stage E0(k+1); issue the loads of E0(k+2), of the codes of plane k+1
-//      and (waves 0, 1) of its iAy / itAy row; E2(k-1) on waves 2..TY+1,
-//      stores; stage E1(k) and the iAy / itAy row; issue the loads of H0(k+1)
+//      and of its metric rows; E2(k-1) on rows 2..T+1, stores; stage E1(k)
+//      and the metric rows; issue the loads of H0(k+1)
 // Loads are in flight during the E2 update before their use, no register is
 // copied from a load before that use, and the per-plane scalars (Lz, tLz, the
-// beam, iAx, itAx) are staged in LDS once per launch, so the waves rarely wait
-// for memory. LDS rows are q-major, so a single-word read takes consecutive
-// words in consecutive lanes (no bank conflicts). E and H are read once and
-// written once per two steps.
+// beam) are staged in LDS once per launch, so the waves rarely wait for
+// memory. LDS holds one block per component and cell of a lane, rows end to
+// end in it, so a single-word read takes consecutive words in consecutive
+// lanes (no bank conflicts). E and H are read once and written once per two
+// steps.
+//
+// What bounds it: the instructions its 12 waves issue (664 of 1,110 a plane are
+// the arithmetic of the exact row sums, FP32), and on large FP32 grids the
+// memory beside it. One branch per update and none per cell, buffer loads that
+// return zeros off the grid, own neighbours from registers: 16% fewer
+// instructions than the first form of this kernel (rows of one wave, a branch
+// per cell). us per step, that form -> this one: 256x256x512 FP32 197 -> 188
+// (1.70 GB per launch at 4.5 TB/s), 200x200x400 FP32 with conduction 149 ->
+// 111, 256x256x128 FP64 134 -> 106; and against one step per launch, which
+// other rows took: 160x160x200 FP64 267 -> 77, 300x220x180 FP32 270 -> 99,
+// 91x75x161 FP32 35 -> 17.6, 48x48x128 FP64 17.2 -> 9.4.
 #pragma once
 #include "step_fused4.h"
 
 namespace wf {
 
-// A read of read-only data through the constant address space: with a uniform
-// index it compiles to a scalar load (SGPR result, scalar cache).
-template <typename T>
-__device__ __forceinline__ T ldc(const T *p, int64_t i) {
-  return ((const __attribute__((address_space(4))) T *)p)[i];
+// One launch of the two-step kernel over a grid.
+struct T2Aux {
+  int ixs, iys;
+  int cap_ix0, cap_iy0, cap_nx, cap_ny;
+  int64_t cap_samples, cap_sample;
+  int KZ, ntx, nty, ntz;  // planes per chunk, tiles
+  int T, OW;              // own rows and cells of a tile
+  int Q, QS;              // lanes and LDS slots of a staged row
+  int l0, ln;             // own lanes of a row: l0 .. l0 + ln - 1, lane l0 at the tile's first cell
+  int skip_j;             // COND: 1 = J is stored by a later launch of the call
+};
+
+// Threads of a workgroup at most, and LDS slots per block of the staged E0, H1,
+// E1, H2 (a buffer of R rows takes R * QS + 1 slots): 144.4 KB of the CU's 160
+constexpr int T2_NT = 768;
+struct T2Slots {
+  static constexpr int E0 = 832, H1 = 768, E1 = 704, H2 = 704;
+};
+
+// An array behind a buffer descriptor: a lane addresses it with a byte offset
+// of its own plus a uniform one (plane and component), so a plane's accesses
+// need no address arithmetic, and a lane whose own offset is OOB reads zeros
+// and writes nothing, so they need no branch.
+constexpr uint32_t OOB = 0xfffffff0u;
+typedef __amdgpu_buffer_rsrc_t Buf;
+__device__ __forceinline__ Buf buf_of(const void *p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00020000);
+}
+template <typename S>
+__device__ __forceinline__ S buf_ld1(Buf b, uint32_t v, uint32_t s) {
+  if constexpr (sizeof(S) == 4) {
+    return __builtin_bit_cast(S, __builtin_amdgcn_raw_buffer_load_b32(b, (int)v, (int)s, 0));
+  } else {
+    return __builtin_bit_cast(S, __builtin_amdgcn_raw_buffer_load_b64(b, (int)v, (int)s, 0));
+  }
+}
+// The byte offsets of a lane's V cells: v for a whole lane; with RAG a lane that
+// the row end cuts has v = OOB and one offset per cell instead.
+template <int V>
+struct Offs {
+  uint32_t v, c[V - 1];
+  bool cut;
+};
+// V cells of each of NC components (cstep bytes apart), 16 bytes at the
+// alignment the row has; zeros unless `in` (uniform: a select costs less here
+// than a branch, which the loads could not be scheduled across)
+template <bool RAG, typename S, int NC, int V>
+__device__ __forceinline__ void buf_ld(Buf b, const Offs<V> &o, bool in, uint32_t s,
+                                       uint32_t cstep, S (&d)[NC][V]) {
+  typedef S vec __attribute__((ext_vector_type(V)));
+  const uint32_t v = in ? o.v : OOB;
+  s = in ? s : 0;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const vec t = __builtin_bit_cast(
+        vec, __builtin_amdgcn_raw_buffer_load_b128(b, (int)v, (int)(s + c * cstep), 0));
+#pragma unroll
+    for (int q = 0; q < V; ++q) d[c][q] = t[q];
+  }
+  if (RAG && o.cut && in) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int q = 0; q < V - 1; ++q) d[c][q] = buf_ld1<S>(b, o.c[q], s + c * cstep);
+  }
+}
+// the same for stores, streamed past the caches (cache policy 2: non-temporal)
+template <bool RAG, typename S, int NC, int V>
+__device__ __forceinline__ void buf_st(Buf b, const Offs<V> &o, uint32_t s, uint32_t cstep,
+                                       const S (&d)[NC][V]) {
+  typedef S vec __attribute__((ext_vector_type(V)));
+  typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    vec t;
+#pragma unroll
+    for (int q = 0; q < V; ++q) t[q] = d[c][q];
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4, t), b, (int)o.v,
+                                           (int)(s + c * cstep), 2);
+  }
+  if (RAG && o.cut) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int q = 0; q < V - 1; ++q) {
+        if constexpr (sizeof(S) == 4)
+          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, d[c][q]), b,
+                                                (int)o.c[q], (int)(s + c * cstep), 2);
+        else
+          __builtin_amdgcn_raw_buffer_store_b64(
+              __builtin_bit_cast(decltype(__builtin_amdgcn_raw_buffer_load_b64(b, 0, 0, 0)),
+                                 d[c][q]),
+              b, (int)o.c[q], (int)(s + c * cstep), 2);
+      }
+  }
 }
 
-template <typename S, bool COND, bool DESC, int TY>
-__global__ void __launch_bounds__(64 * (TY + 4) * (int)(sizeof(S) / 4))
-k_fused4_t2(GridDev g, MetricDev<S> m, const S *__restrict__ Ein, const S *__restrict__ Hin,
-            S *__restrict__ Eout, S *__restrict__ Hout, S *__restrict__ J, Coefs<S> cf, S dt,
-            FusedAux x, const S *__restrict__ beam1, const S *__restrict__ beam2,
-            S *__restrict__ cap) {
+// Dynamic LDS of a workgroup in values of S: the ring of iAy / itAy rows, the
+// x metric, the ring of iAx / itAx values, the per-plane scalars, the material
+// table.
+__host__ __device__ inline int t2_dyn_values(int V, int Q, int T, int KZ, int nmat) {
+  return 8 * Q * V + 6 * (T + 4) + 4 * (KZ + 3) + 9 * nmat;
+}
+
+template <typename S, bool COND, bool DESC, bool RAG>
+__device__ __forceinline__ void
+t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
+        const S *__restrict__ Hin, S *__restrict__ Eout, S *__restrict__ Hout,
+        S *__restrict__ J, const Coefs<S> &cf, S dt, const T2Aux &x,
+        const S *__restrict__ beam1, const S *__restrict__ beam2, S *__restrict__ cap,
+        const int tile) {
   using I = uint32_t;  // byte offsets: every 3N array within 4 GiB
   constexpr int V = 16 / sizeof(S);
-  constexpr int WPR = sizeof(S) / 4;  // waves per row: 1 FP32, 2 FP64
-  constexpr int LR = 64 * WPR;        // lanes per row
-  constexpr int W = LR * V;           // cells per row (256)
-  // LDS rows are q-major: the cell V*ln+q of row lane ln at slot q*QS + ln + 1,
-  // so that one value per lane is LR consecutive words (no bank conflicts for
-  // the single-word reads of the x neighbours and of cells one at a time).
-  // Slot 0 of block V-1 is cell -1 and slot QS-1 of block 0 is cell W: both
-  // stay 0.
-  constexpr int QS = LR + 2;
-  constexpr int RW = V * QS;
   constexpr int NM = 9;
-  constexpr int RE0 = TY + 4, RH1 = TY + 3, RE1 = TY + 2, RH2 = TY + 1;
-  constexpr int NT = 64 * (TY + 4) * WPR;
-  __shared__ S sE0_[3 * RE0 * RW];  // E0(k), rows j0-2 .. j0+TY+1
-  __shared__ S sH1_[3 * RH1 * RW];  // H1(k), rows j0-2 .. j0+TY
-  __shared__ S sE1_[3 * RE1 * RW];  // E1(k-1) until P3 stages E1(k), rows j0-1 .. j0+TY
-  __shared__ S sH2_[3 * RH2 * RW];  // H2(k-1), rows j0-1 .. j0+TY-1
-  // iAy and itAy of planes k-1, k, k+1 (slot plane % 3), lane-major, written
-  // by waves 0 and 1
-  __shared__ __attribute__((aligned(16))) S sCy_[3 * 2 * W];
-  extern __shared__ unsigned char s_dyn[];
-  S *sMat = reinterpret_cast<S *>(s_dyn);
-  const auto sE0 = [&](int c, int r) { return sE0_ + (c * RE0 + r) * RW; };
-  const auto sH1 = [&](int c, int r) { return sH1_ + (c * RH1 + r) * RW; };
-  const auto sE1 = [&](int c, int r) { return sE1_ + (c * RE1 + r) * RW; };
-  const auto sH2 = [&](int c, int r) { return sH2_ + (c * RH2 + r) * RW; };
-  const auto sCy = [&](int kk, int which) { return sCy_ + (((kk + 3) % 3) * 2 + which) * W; };
+  constexpr int CE0 = T2Slots::E0, CH1 = T2Slots::H1, CE1 = T2Slots::E1, CH2 = T2Slots::H2;
+  // blocks [component][cell of the lane][slot]; the slot of lane ln of row r is
+  // r * QS + ln + 1; a slot that no lane owns stays 0. Of H_y only the last
+  // cell of a lane is read by another one: one block.
+  __shared__ S sE0_[3 * V * CE0];        // E0(k), rows j0-2 .. j0+T+1
+  __shared__ S sH1_[(2 * V + 1) * CH1];  // H1(k), rows j0-2 .. j0+T
+  __shared__ S sE1_[3 * V * CE1];        // E1(k-1) until P3 stages E1(k), rows j0-1 .. j0+T
+  __shared__ S sH2_[(2 * V + 1) * CH2];  // H2(k-1), rows j0-1 .. j0+T-1
+  extern __shared__ __align__(16) unsigned char s_dyn[];
+  const int Q = x.Q, QS = x.QS, T = x.T;
+  S *sCy = reinterpret_cast<S *>(s_dyn);  // [plane % 3][iAy, itAy][Q * V]
+  S *sX = sCy + 3 * 2 * Q * V;            // [Lx, tLx][Q * V]
+  S *sRow = sX + 2 * Q * V;               // [plane % 3][iAx, itAx][T + 4]
+  S *sPl = sRow + 3 * 2 * (T + 4);        // [Lz, tLz, beam 1, beam 2][KZ + 3]
+  S *sMat = sPl + 4 * (x.KZ + 3);         // [nmat][9]
   typedef S vec __attribute__((ext_vector_type(V)));
   const auto ldsv = [&](const S *p, S (&o)[V]) {
     const vec v = *reinterpret_cast<const vec *>(p);
@@ -83,88 +192,113 @@ k_fused4_t2(GridDev g, MetricDev<S> m, const S *__restrict__ Ein, const S *__res
     for (int q = 0; q < V; ++q) o[q] = v[q];
   };
 
-  for (int t = threadIdx.x; t < cf.nmat * NM; t += NT) sMat[t] = cf.mat[t];
-  // the x-halo slots (cells -1 and W) are zero for the whole launch
-  for (int t = threadIdx.x; t < 3 * (RE0 + RH1 + RE1 + RH2) * 2; t += NT) {
-    int r = t >> 1;  // component row over the four buffers
-    const int slot = (t & 1) ? QS - 1 : (V - 1) * QS;
-    S *base;
-    if (r < 3 * RE0) {
-      base = sE0_;
-    } else if ((r -= 3 * RE0) < 3 * RH1) {
-      base = sH1_;
-    } else if ((r -= 3 * RH1) < 3 * RE1) {
-      base = sE1_;
-    } else {
-      r -= 3 * RE1;
-      base = sH2_;
-    }
-    base[r * RW + slot] = S(0);
-  }
-
-  const int tile = xcd_tile(blockIdx.x, x.nty * x.ntz);
-  const int tz = tile / x.nty, ty = tile - tz * x.nty;
-  const int j0 = ty * TY, k0 = tz * x.KZ;
-  const int kend = min(k0 + x.KZ, g.Nz);
-  // the row of a wave is uniform: row flags, row metrics and branches are scalar
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int w = wave / WPR;                              // row of the workgroup
-  const int ln = (wave - w * WPR) * 64 + (threadIdx.x & 63);  // lane in the row
-  const int j = j0 - 2 + w;
-  const bool rowok = (j >= 0) && (j < g.Ny);
-  const int xi = V * ln;
-  // LDS slot of cell xi + q, -1 <= q <= V (q is a constant after unrolling)
-  const auto atx = [&](int q) {
-    return q < 0 ? (V - 1) * QS + ln : q >= V ? ln + 2 : q * QS + ln + 1;
-  };
-  const bool lact = rowok && (xi < g.Nx);
-  const I N = (I)g.N, sz = (I)g.sz;
-  const I col = lact ? (I)xi + (I)g.sy * (I)j : (I)0;
-  const bool doH1 = w <= TY + 2, doE1 = w >= 1 && w <= TY + 2;
-  const bool doH2 = w >= 1 && w <= TY + 1, own = w >= 2 && w <= TY + 1;
-
-  S Lx[V], tLx[V], iAz[V], itAz[V];
+  for (int t = threadIdx.x; t < cf.nmat * NM; t += blockDim.x) sMat[t] = cf.mat[t];
+  // the slots that no lane owns: the one before the first row, and the gaps
+  for (int t = threadIdx.x; t <= (QS > Q ? T + 4 : 0); t += blockDim.x) {
+    const int s = t * QS;
 #pragma unroll
-  for (int q = 0; q < V; ++q) {
-    Lx[q] = lact ? m.Lx[xi + q] : S(0);
-    tLx[q] = lact ? m.tLx[xi + q] : S(0);
-    iAz[q] = S(0);
-    itAz[q] = S(0);
+    for (int b = 0; b < 3 * V; ++b) {
+      if (t <= T + 4) sE0_[b * CE0 + s] = S(0);
+      if (b < 2 * V + 1 && t <= T + 3) sH1_[b * CH1 + s] = S(0);
+      if (t <= T + 2) sE1_[b * CE1 + s] = S(0);
+      if (b < 2 * V + 1 && t <= T + 1) sH2_[b * CH2 + s] = S(0);
+    }
   }
-  if (lact) {
-    const I o = (I)xi + (I)g.Nx * (I)j;
-    ldv<V>(cf.iAz, o, iAz);
-    ldv<V>(cf.itAz, o, itAz);
+
+  const int tx = tile % x.ntx, tyz = tile / x.ntx;
+  const int tz = tyz / x.nty, ty = tyz - tz * x.nty;
+  const int j0 = ty * T, k0 = tz * x.KZ;
+  const int kend = min(k0 + x.KZ, g.Nz);
+  const int r = (int)threadIdx.x / Q;  // row of the workgroup
+  const int ln = (int)threadIdx.x - r * Q;
+  const bool act = r < T + 4;
+  const int j = j0 - 2 + r;
+  const bool rowok = act && (j >= 0) && (j < g.Ny);
+  const int xi = tx * x.OW + V * (ln - x.l0);
+  // cells of this lane inside the row
+  const int nvx = (xi >= 0 && xi < g.Nx) ? (RAG ? min(V, g.Nx - xi) : V) : 0;  // of any row
+  const int nv = rowok ? nvx : 0;
+  const bool lact = nv > 0;
+  const I ES = (I)sizeof(S), NB = (I)g.N * ES, sz = (I)g.sz;
+  const I cell = lact ? (I)xi + (I)g.sy * (I)j : (I)0;  // in its plane
+  const bool doH1 = r <= T + 2, doE1 = r >= 1 && r <= T + 2;
+  const bool doH2 = r >= 1 && r <= T + 1;
+  const bool own = lact && r >= 2 && r <= T + 1 && ln >= x.l0 && ln < x.l0 + x.ln;
+  // byte offsets of this lane's cells in a plane
+  const auto offs = [&](int n, I at_cell, bool on) {
+    Offs<V> o;
+    o.v = (on && n == V) ? at_cell * ES : OOB;
+    o.cut = RAG && on && n > 0 && n < V;
+#pragma unroll
+    for (int q = 0; q < V - 1; ++q) o.c[q] = (o.cut && q < n) ? (at_cell + (I)q) * ES : OOB;
+    return o;
+  };
+  const Offs<V> of = offs(nv, cell, true);
+  Offs<V> ofh = of, ofs = of;  // H0 (not read on the last row); stores
+  if (!doH1) ofh.v = OOB;
+  if (!own) {
+    ofs.v = OOB;
+    ofs.cut = false;
   }
-  const S Ly = rowok ? ldc(m.Ly, j) : S(0), tLy = rowok ? ldc(m.tLy, j) : S(0);
-  const int qbeam = (lact && j == x.iys && x.ixs >= xi && x.ixs < xi + V) ? x.ixs - xi : -1;
-  // Ez window capture: own rows only, one sample per level
+  const I vc = (doH1 && nv == V) ? cell : OOB;                 // codes
+  // the 2-D metric tables lie in one array, iAx first: rows 0 and 1 read the
+  // iAy and itAy of their cells, the first lane of a row its iAx and itAx
+  const I yz = (I)g.Ny * (I)g.Nz, xz = (I)g.Nx * (I)g.Nz, xy = (I)g.Nx * (I)g.Ny;
+  const Offs<V> ofy = offs(r < 2 ? nvx : 0, (I)xi + (r == 0 ? yz : 2 * yz + xz + xy), r < 2);
+  const I vx = (ln == 0 && rowok) ? (I)j * ES : OOB;
+  const Buf bEi = buf_of(Ein, 3 * NB), bHi = buf_of(Hin, 3 * NB);
+  const Buf bEo = buf_of(Eout, 3 * NB), bHo = buf_of(Hout, 3 * NB);
+  const Buf bC = buf_of(cf.code, (I)g.N), bM = buf_of(cf.iAx, 2 * (yz + xz + xy) * ES);
+  // slots of this lane: own row in E0 and H1 (P), the rows of the other buffers
+  // start one row later
+  const int P = r * QS + ln + 1, Pu = P + QS, Pd = P - QS, Pdd = Pd - QS;
+  // cell xi + q (0 <= q <= V) of component c at slot s of a buffer
+  const auto e0 = [&](int c, int s, int q) -> S & {
+    return q >= V ? sE0_[(c * V) * CE0 + s + 1] : sE0_[(c * V + q) * CE0 + s];
+  };
+  const auto e1 = [&](int c, int s, int q) -> S & {
+    return q >= V ? sE1_[(c * V) * CE1 + s + 1] : sE1_[(c * V + q) * CE1 + s];
+  };
+  // blocks of H: x, z, then the last cell of y
+  const auto hb = [](int c, int q) { return c == 0 ? q : c == 2 ? V + q : 2 * V; };
+  const auto h1 = [&](int c, int s, int q) -> S & { return sH1_[hb(c, q) * CH1 + s]; };
+  const auto h2 = [&](int c, int s, int q) -> S & { return sH2_[hb(c, q) * CH2 + s]; };
+
+  if (r < 2) {
+#pragma unroll
+    for (int q = 0; q < V; ++q)
+      sX[(r * Q + ln) * V + q] = q < nvx ? (r == 0 ? m.Lx : m.tLx)[xi + q] : S(0);
+  }
+  S iAz[1][V], itAz[1][V];
+  buf_ld<RAG>(bM, of, true, (yz + xz) * ES, 0, iAz);
+  buf_ld<RAG>(bM, of, true, (2 * (yz + xz) + xy) * ES, 0, itAz);
+  const S Ly = rowok ? m.Ly[j] : S(0), tLy = rowok ? m.tLy[j] : S(0);
+  const int qbeam = (lact && j == x.iys && x.ixs >= xi && x.ixs < xi + nv) ? x.ixs - xi : -1;
+  // Ez window capture: own cells only, one sample per level
   int capq0 = V, capq1 = 0;
-  int64_t capb1 = 0, capb2 = 0;
-  if (cap && own && lact && j >= x.cap_iy0 && j < x.cap_iy0 + x.cap_ny) {
-    const int lo = max(xi, x.cap_ix0), hi = min(xi + V, x.cap_ix0 + x.cap_nx);
+  int64_t capb1 = 0;
+  if (cap && own && j >= x.cap_iy0 && j < x.cap_iy0 + x.cap_ny) {
+    const int lo = max(xi, x.cap_ix0), hi = min(xi + nv, x.cap_ix0 + x.cap_nx);
     if (lo < hi) {
       capq0 = lo - xi; capq1 = hi - xi;
       capb1 = ((int64_t)(j - x.cap_iy0) * x.cap_samples + x.cap_sample) * g.Nz;
-      capb2 = capb1 + g.Nz;
     }
   }
-  const bool cap1 = x.cap_sample < x.cap_samples, cap2 = x.cap_sample + 1 < x.cap_samples;
-  const int64_t capl = (int64_t)x.cap_ny * x.cap_samples * g.Nz;  // stride of one x line
+  const auto capture = [&](int64_t at_plane, const S (&ez)[V]) {
+    const int64_t capl = (int64_t)x.cap_ny * x.cap_samples * g.Nz;  // stride of one x line
+#pragma unroll
+    for (int q = 0; q < V; ++q)
+      if (q >= capq0 && q < capq1) cap[capb1 + at_plane + (int64_t)(q + xi - x.cap_ix0) * capl] = ez[q];
+  };
 
   const int kstart = max(k0 - 2, 0);
-  const int kE1 = max(k0 - 1, 0);  // first plane with E1 (and H2)
-  // per-plane values of planes kstart .. kend, staged once (no scalar memory
-  // load in the z-march: its out-of-order return would make every LDS wait
-  // also wait for it): Lz, tLz, the beam of both levels, and iAx, itAx of the
-  // workgroup's rows
-  const int NP = kend - kstart + 1;
-  S *sPl = sMat + cf.nmat * NM;     // [4][NP]
-  S *sRow = sPl + 4 * NP;           // [2][TY+4][NP]
-  for (int t = threadIdx.x; t < 4 * NP; t += NT) {
+  // per-plane values of planes kstart .. kend, staged once: Lz, tLz, the beam
+  // of both levels
+  const int NP = x.KZ + 3;
+  for (int t = threadIdx.x; t < 4 * NP; t += blockDim.x) {
     const int which = t / NP, kk = kstart + t - which * NP;
     S v = S(0);
-    if (kk < g.Nz) {
+    if (kk < g.Nz && kk <= kend) {
       if (which == 0) v = m.Lz[kk];
       else if (which == 1) v = m.tLz[kk];
       else if (which == 2) v = beam1 ? beam1[kk] : S(0);
@@ -172,215 +306,187 @@ k_fused4_t2(GridDev g, MetricDev<S> m, const S *__restrict__ Ein, const S *__res
     }
     sPl[t] = v;
   }
-  for (int t = threadIdx.x; t < 2 * (TY + 4) * NP; t += NT) {
-    const int which = t / ((TY + 4) * NP), rem = t - which * (TY + 4) * NP;
-    const int r = rem / NP, kk = kstart + rem - r * NP, jj = j0 - 2 + r;
-    S v = S(0);
-    if (jj >= 0 && jj < g.Ny && kk < g.Nz)
-      v = (which ? cf.itAx : cf.iAx)[(int64_t)jj + (int64_t)g.Ny * kk];
-    sRow[t] = v;
-  }
   const auto plv = [&](int which, int kk) { return sPl[which * NP + kk - kstart]; };
-  const auto rowv = [&](int which, int kk) {
-    return sRow[(which * (TY + 4) + w) * NP + kk - kstart];
+  const auto ring = [](int kk) { return (kk + 3) % 3; };
+  const auto rowv = [&](int which, int slot) { return sRow[(slot * 2 + which) * (T + 4) + r]; };
+  const auto cyv = [&](int which, int slot) { return sCy + ((slot * 2 + which) * Q + ln) * V; };
+  // planes past the grid are zeros
+  const auto load_e = [&](int kk, S (&o)[3][V]) {
+    buf_ld<RAG>(bEi, of, kk < g.Nz, (I)kk * sz * ES, NB, o);
   };
-  S Ek[3][V], Ek1[3][V];
+  const auto load_h = [&](int kk, S (&o)[3][V]) {
+    buf_ld<RAG>(bHi, ofh, kk < g.Nz, (I)kk * sz * ES, NB, o);
+  };
+  const auto load_code = [&](int kk) -> uint32_t {
+    const bool in = kk < g.Nz;
+    const int v = (int)(in ? vc : OOB), s = in ? (int)((I)kk * sz) : 0;
+    uint32_t c;
+    if constexpr (V == 4) c = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(bC, v, s, 0);
+    else c = (uint32_t)(uint16_t)__builtin_amdgcn_raw_buffer_load_b16(bC, v, s, 0);
+    if (RAG && of.cut && in) {
+      c = 0;
 #pragma unroll
-  for (int c = 0; c < 3; ++c)
-#pragma unroll
-    for (int q = 0; q < V; ++q) { Ek[c][q] = S(0); Ek1[c][q] = S(0); }
-  if (lact) {
-    const I n = col + sz * (I)kstart;
-    ldv<V>(Ein, n, Ek[0]); ldv<V>(Ein, N + n, Ek[1]); ldv<V>(Ein, 2 * N + n, Ek[2]);
-    if (kstart + 1 < g.Nz) {
-      ldv<V>(Ein, n + sz, Ek1[0]); ldv<V>(Ein, N + n + sz, Ek1[1]);
-      ldv<V>(Ein, 2 * N + n + sz, Ek1[2]);
+      for (int q = 0; q < V - 1; ++q)
+        c |= (uint32_t)(uint8_t)__builtin_amdgcn_raw_buffer_load_b8(
+                 bC, (int)(q < nv ? cell + (I)q : OOB), s, 0) << (8 * q);
     }
-  }
-  // carried between planes: H1(k-1), H2(k-2) (x, y) and the codes of plane
-  // k-1 (level 2's coefficients; its metric values come from the tables)
-  S H1p[3][V], H2p[2][V];
-#pragma unroll
-  for (int q = 0; q < V; ++q) {
-    H1p[0][q] = H1p[1][q] = H1p[2][q] = S(0);
-    H2p[0][q] = H2p[1][q] = S(0);
-  }
-  uint32_t codep = 0;
-  // the plane in hand, loaded one plane ahead: H0 and the codes; waves 0 and 1
-  // also carry its iAy / itAy row on the way to sCy
-  struct Plane {
-    S h[3][V], cy[V];
-    uint32_t code;
+    return c;
   };
-  // iAy / itAy of plane kk (issued early: few registers)
-  const auto load_plane_a = [&](int kk, Plane &P) {
-#pragma unroll
-    for (int q = 0; q < V; ++q) P.cy[q] = S(0);
-    if (kk < g.Nz && w < 2 && xi < g.Nx)
-      ldv<V>(w == 0 ? cf.iAy : cf.itAy, (I)xi + (I)g.Nx * (I)kk, P.cy);
+  struct Row {
+    S cy[1][V], ax, bx;
   };
-  // the codes of plane kk
-  const auto load_code = [&](int kk, Plane &P) {
-    P.code = (kk < g.Nz && lact && doH1) ? ldcode<V>(cf.code, col + sz * (I)kk) : 0u;
+  // the metric rows of plane kk, and their place in the rings
+  const auto load_row = [&](int kk, Row &o) {
+    const bool in = kk < g.Nz;
+    buf_ld<RAG>(bM, ofy, in, (I)kk * (I)g.Nx * ES, 0, o.cy);
+    const I v = in ? vx : OOB, s = in ? (I)kk * (I)g.Ny * ES : 0;
+    o.ax = buf_ld1<S>(bM, v, s);
+    o.bx = buf_ld1<S>(bM, v, s + (yz + xz + xy) * ES);
   };
-  // H0 of plane kk (issued last: its registers live until H1)
-  const auto load_plane_b = [&](int kk, Plane &P) {
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-      for (int q = 0; q < V; ++q) P.h[c][q] = S(0);
-    if (kk < g.Nz && lact && doH1) {
-      const I n = col + sz * (I)kk;
-      ldv<V>(Hin, n, P.h[0]); ldv<V>(Hin, N + n, P.h[1]); ldv<V>(Hin, 2 * N + n, P.h[2]);
-    }
-  };
-  const auto put_ring = [&](int kk, const Plane &P) {
-    if (w < 2 && kk <= g.Nz) {
+  const auto put_row = [&](int kk, const Row &o) {
+    const int slot = ring(kk);
+    if (r < 2) {
       vec v;
 #pragma unroll
-      for (int q = 0; q < V; ++q) v[q] = P.cy[q];
-      *reinterpret_cast<vec *>(sCy(kk, w) + xi) = v;
+      for (int q = 0; q < V; ++q) v[q] = o.cy[0][q];
+      *reinterpret_cast<vec *>(cyv(r, slot)) = v;
+    }
+    if (ln == 0 && act) {
+      sRow[(slot * 2 + 0) * (T + 4) + r] = o.ax;
+      sRow[(slot * 2 + 1) * (T + 4) + r] = o.bx;
     }
   };
-  Plane P;
-  load_plane_a(kstart, P);
-  load_code(kstart, P);
-  load_plane_b(kstart, P);
-  put_ring(kstart, P);
+
+  S Ek1[3][V], h0[3][V];  // E0(k+1), H0(k)
+  uint32_t code = load_code(kstart), codep = 0;
+  {
+    S Ek[3][V];
+    Row row;
+    load_e(kstart, Ek);
+    load_row(kstart, row);
+    load_e(kstart + 1, Ek1);
+    load_h(kstart, h0);
+    if (act) {
 #pragma unroll
-  for (int c = 0; c < 3; ++c)
+      for (int c = 0; c < 3; ++c)
 #pragma unroll
-    for (int q = 0; q < V; ++q) sE0(c, w)[atx(q)] = lact ? Ek[c][q] : S(0);
+        for (int q = 0; q < V; ++q) e0(c, P, q) = Ek[c][q];
+    }
+    put_row(kstart, row);
+  }
+  // carried between planes: H1(k-1), H2(k-2) (x, y) and the codes of plane
+  // k-1 (level 2's coefficients; its metric values come from the rings). A
+  // lane outside the grid holds zeros: its fields and metric values are 0.
+  S H1[3][V], E1[3][V], H2[3][V], H1p[3][V], H2p[2][V];
+#pragma unroll
+  for (int q = 0; q < V; ++q) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) H1[c][q] = E1[c][q] = H2[c][q] = H1p[c][q] = S(0);
+    H2p[0][q] = H2p[1][q] = S(0);
+  }
   __syncthreads();
 
   for (int k = kstart; k <= kend; ++k) {
-    const bool pl1 = k < g.Nz;                // level-1 plane exists
-    const int p = k - 1;                      // level-2 plane
-    const bool l2h = p >= kE1 && p < kend;    // H2(p) needed
-    const bool l2e = p >= k0 && p < kend;     // E2(p) stored
-    const uint32_t code = P.code;
-    const S iax = rowv(0, k), itax = rowv(1, k), Lz = plv(0, k), tLz = plv(1, k);
-    const int pp = max(p, kstart);  // level 2 reads only for p >= kE1 >= kstart
-    const S iaxp = rowv(0, pp), itaxp = rowv(1, pp), Lzp = plv(0, pp), tLzp = plv(1, pp);
+    const int p = k - 1;                   // level-2 plane
+    const bool l2e = p >= k0 && p < kend;  // E2(p) and H2(p) stored
+    const int rk = ring(k), rp = ring(p);
 
     // ---- P1: H1(k)
-    S H1[3][V];
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-      for (int q = 0; q < V; ++q) H1[c][q] = S(0);
-    if (lact && pl1 && doH1) {
-      S c0y[V];
-      ldsv(sCy(k, 0) + xi, c0y);
-      S EX[V + 1], EY[V + 1], EZ[V + 1];
+    if (doH1) {
+      const S iax = rowv(0, rk), Lz = plv(0, k);
+      S c0y[V], Lx[V];
+      ldsv(cyv(0, rk), c0y);
+      ldsv(sX + ln * V, Lx);
+      S EX[V], EY[V + 1], EZ[V + 1];
 #pragma unroll
       for (int q = 0; q < V + 1; ++q) {
-        EX[q] = sE0(0, w)[atx(q)]; EY[q] = sE0(1, w)[atx(q)];
-        EZ[q] = sE0(2, w)[atx(q)];
+        if (q < V) EX[q] = e0(0, P, q);
+        EY[q] = e0(1, P, q); EZ[q] = e0(2, P, q);
       }
 #pragma unroll
       for (int q = 0; q < V; ++q) {
         const S *t = sMat + NM * (int)((code >> (8 * q)) & 0xffu);
-        const S a0 = (S)(iax * t[0]), a1 = (S)(c0y[q] * t[1]), a2 = (S)(iAz[q] * t[2]);
-        H1[0][q] = h_row<S, S, DESC>(P.h[0][q], a0, dt, Ly, Lz, EY[q], Ek1[1][q], EZ[q],
-                                     sE0(2, w + 1)[atx(q)], +1, -1);
-        H1[1][q] = h_row<S, S, DESC>(P.h[1][q], a1, dt, Lx[q], Lz, EX[q], Ek1[0][q], EZ[q],
+        const S a0 = (S)(iax * t[0]), a1 = (S)(c0y[q] * t[1]), a2 = (S)(iAz[0][q] * t[2]);
+        H1[0][q] = h_row<S, S, DESC>(h0[0][q], a0, dt, Ly, Lz, EY[q], Ek1[1][q], EZ[q],
+                                     e0(2, Pu, q), +1, -1);
+        H1[1][q] = h_row<S, S, DESC>(h0[1][q], a1, dt, Lx[q], Lz, EX[q], Ek1[0][q], EZ[q],
                                      EZ[q + 1], -1, +1);
-        H1[2][q] = h_row<S, S, DESC>(P.h[2][q], a2, dt, Lx[q], Ly, EX[q],
-                                     sE0(0, w + 1)[atx(q)], EY[q], EY[q + 1], +1, -1);
+        H1[2][q] = h_row<S, S, DESC>(h0[2][q], a2, dt, Lx[q], Ly, EX[q],
+                                     e0(0, Pu, q), EY[q], EY[q + 1], +1, -1);
+        h1(0, P, q) = H1[0][q];
+        h1(2, P, q) = H1[2][q];
+        if (q == V - 1) h1(1, P, q) = H1[1][q];
       }
-    }
-    if (doH1) {
-#pragma unroll
-      for (int c = 0; c < 3; ++c)
-#pragma unroll
-        for (int q = 0; q < V; ++q) sH1(c, w)[atx(q)] = H1[c][q];
     }
     __syncthreads();
 
     // ---- P2: E1(k), then H2(k-1)
-    S E1[3][V];
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-      for (int q = 0; q < V; ++q) E1[c][q] = S(0);
-    if (lact && pl1 && doE1 && k >= kE1) {
-      S c1y[V];
-      ldsv(sCy(k, 1) + xi, c1y);
-      S HX[V + 1], HY[V + 1], HZ[V + 1];  // [0] = -x neighbour
-#pragma unroll
-      for (int q = 0; q < V + 1; ++q) {
-        HX[q] = sH1(0, w)[atx(q - 1)];
-        HY[q] = sH1(1, w)[atx(q - 1)];
-        HZ[q] = sH1(2, w)[atx(q - 1)];
-      }
+    if (doE1) {
+      const S itax = rowv(1, rk), tLz = plv(1, k), bm = plv(2, k);
+      S c1y[V], tLx[V];
+      ldsv(cyv(1, rk), c1y);
+      ldsv(sX + (Q + ln) * V, tLx);
+      const S HYm = h1(1, P - 1, V - 1), HZm = h1(2, P - 1, V - 1);  // -x neighbours
+      S s2[V];
 #pragma unroll
       for (int q = 0; q < V; ++q) {
         const S *t = sMat + NM * (int)((code >> (8 * q)) & 0xffu);
-        const S b0 = (S)(t[3] * itax), b1 = (S)(t[4] * c1y[q]), b2 = (S)(t[5] * itAz[q]);
-        S d0 = e_sum<S>(b0, tLy, tLz, H1p[1][q], HY[q + 1], sH1(2, w - 1)[atx(q)],
-                        HZ[q + 1], +1, -1);
-        S d1 = e_sum<S>(b1, tLx[q], tLz, H1p[0][q], HX[q + 1], HZ[q], HZ[q + 1], -1, +1);
-        S d2 = e_sum<S>(b2, tLx[q], tLy, sH1(0, w - 1)[atx(q)], HX[q + 1], HY[q],
-                        HY[q + 1], +1, -1);
-        const S e0 = sE0(0, w)[atx(q)], e1 = sE0(1, w)[atx(q)];
-        const S e2 = sE0(2, w)[atx(q)];  // E0(k) as staged
-        if (COND) {  // J = sigma E0 (the beam's current on its line)
-          d0 = d0 - t[3] * (S)(t[6] * e0);
-          d1 = d1 - t[4] * (S)(t[7] * e1);
-          d2 = d2 - t[5] * ((q == qbeam) ? plv(2, k) : (S)(t[8] * e2));
-        } else if (q == qbeam) {
-          d2 = d2 - t[5] * plv(2, k);
+        const S b0 = (S)(t[3] * itax), b1 = (S)(t[4] * c1y[q]), b2 = (S)(t[5] * itAz[0][q]);
+        S d0 = e_sum<S>(b0, tLy, tLz, H1p[1][q], H1[1][q], h1(2, Pd, q), H1[2][q], +1, -1);
+        S d1 = e_sum<S>(b1, tLx[q], tLz, H1p[0][q], H1[0][q], q ? H1[2][q - 1] : HZm, H1[2][q],
+                        -1, +1);
+        S d2 = e_sum<S>(b2, tLx[q], tLy, h1(0, Pd, q), H1[0][q], q ? H1[1][q - 1] : HYm,
+                        H1[1][q], +1, -1);
+        s2[q] = d2;
+        const S o0 = e0(0, P, q), o1 = e0(1, P, q), o2 = e0(2, P, q);  // E0(k) as staged
+        if (COND) {  // J = sigma E0
+          d0 = d0 - t[3] * (S)(t[6] * o0);
+          d1 = d1 - t[4] * (S)(t[7] * o1);
+          d2 = d2 - t[5] * (S)(t[8] * o2);
         }
-        E1[0][q] = (S)(e0 + dt * d0);
-        E1[1][q] = (S)(e1 + dt * d1);
-        E1[2][q] = (S)(e2 + dt * d2);
-        if (cap1 && k >= k0 && k < kend && q >= capq0 && q < capq1)
-          cap[capb1 + (int64_t)(q + xi - x.cap_ix0) * capl + k] = E1[2][q];
+        E1[0][q] = (S)(o0 + dt * d0);
+        E1[1][q] = (S)(o1 + dt * d1);
+        E1[2][q] = (S)(o2 + dt * d2);
       }
+      if (qbeam >= 0) {  // the beam's current instead on its line
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+          const S *t = sMat + NM * (int)((code >> (8 * q)) & 0xffu);
+          const S d2 = s2[q] - t[5] * bm;
+          if (q == qbeam) E1[2][q] = (S)(e0(2, P, q) + dt * d2);
+        }
+      }
+      if (capq0 < capq1 && x.cap_sample < x.cap_samples && k >= k0 && k < kend)
+        capture(k, E1[2]);
     }
-    S H2[3][V];
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-      for (int q = 0; q < V; ++q) H2[c][q] = S(0);
-    if (lact && doH2 && l2h) {
-      S c0yp[V];
-      ldsv(sCy(p, 0) + xi, c0yp);
-      // E1(p): own row from sE1 row w-1 (x neighbour in slot q = V), row j+1 from row w
-      S EX[V + 1], EY[V + 1], EZ[V + 1];
+    if (doH2 && p >= kstart) {  // H2 below plane 0 stays 0
+      const S iaxp = rowv(0, rp), Lzp = plv(0, p);
+      S c0yp[V], Lx[V];
+      ldsv(cyv(0, rp), c0yp);
+      ldsv(sX + ln * V, Lx);
+      // E1(p): own row from slot Pd (x neighbour at q = V), row j+1 from slot P
+      S EX[V], EY[V + 1], EZ[V + 1];
 #pragma unroll
       for (int q = 0; q < V + 1; ++q) {
-        EX[q] = sE1(0, w - 1)[atx(q)]; EY[q] = sE1(1, w - 1)[atx(q)];
-        EZ[q] = sE1(2, w - 1)[atx(q)];
+        if (q < V) EX[q] = e1(0, Pd, q);
+        EY[q] = e1(1, Pd, q); EZ[q] = e1(2, Pd, q);
       }
 #pragma unroll
       for (int q = 0; q < V; ++q) {
         const S *t = sMat + NM * (int)((codep >> (8 * q)) & 0xffu);
-        const S a0 = (S)(iaxp * t[0]), a1 = (S)(c0yp[q] * t[1]), a2 = (S)(iAz[q] * t[2]);
+        const S a0 = (S)(iaxp * t[0]), a1 = (S)(c0yp[q] * t[1]), a2 = (S)(iAz[0][q] * t[2]);
         H2[0][q] = h_row<S, S, DESC>(H1p[0][q], a0, dt, Ly, Lzp, EY[q], E1[1][q], EZ[q],
-                                     sE1(2, w)[atx(q)], +1, -1);
+                                     e1(2, P, q), +1, -1);
         H2[1][q] = h_row<S, S, DESC>(H1p[1][q], a1, dt, Lx[q], Lzp, EX[q], E1[0][q], EZ[q],
                                      EZ[q + 1], -1, +1);
         H2[2][q] = h_row<S, S, DESC>(H1p[2][q], a2, dt, Lx[q], Ly, EX[q],
-                                     sE1(0, w)[atx(q)], EY[q], EY[q + 1], +1, -1);
+                                     e1(0, P, q), EY[q], EY[q + 1], +1, -1);
+        h2(0, Pd, q) = H2[0][q];
+        h2(2, Pd, q) = H2[2][q];
+        if (q == V - 1) h2(1, Pd, q) = H2[1][q];
       }
-    }
-    if (doH2) {
-#pragma unroll
-      for (int c = 0; c < 3; ++c)
-#pragma unroll
-        for (int q = 0; q < V; ++q) sH2(c, w - 1)[atx(q)] = H2[c][q];
-    }
-    // H2(k-1) of the own rows is final: stored now; its x, y components are
-    // kept for E2(k) of the next plane
-    S H2c[2][V];
-#pragma unroll
-    for (int q = 0; q < V; ++q) { H2c[0][q] = H2[0][q]; H2c[1][q] = H2[1][q]; }
-    if (lact && own && l2e) {
-      const I np = col + sz * (I)p;
-      stv_nt<V>(Hout, np, H2[0]); stv_nt<V>(Hout, N + np, H2[1]);
-      stv_nt<V>(Hout, 2 * N + np, H2[2]);
+      // H2(k-1) of the own rows is final
+      if (l2e) buf_st<RAG>(bHo, ofs, (I)p * sz * ES, NB, H2);
     }
 #pragma unroll
     for (int c = 0; c < 3; ++c)
@@ -390,83 +496,91 @@ k_fused4_t2(GridDev g, MetricDev<S> m, const S *__restrict__ Ein, const S *__res
 
     // ---- P3: stage E0(k+1) (sE0 is free once E1(k) is done); loads of plane
     // k+1 and of E0(k+2); E2(k-1) on the own rows, stores; stage E1(k)
-    const bool more = k < kend;
-    const S bv2 = plv(3, pp);  // the beam at plane p, level 2
+    if (act) {
 #pragma unroll
-    for (int c = 0; c < 3; ++c)
+      for (int c = 0; c < 3; ++c)
 #pragma unroll
-      for (int q = 0; q < V; ++q) sE0(c, w)[atx(q)] = Ek1[c][q];
-    load_plane_a(more ? k + 1 : g.Nz + 1, P);
-    load_code(more ? k + 1 : g.Nz, P);
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-      for (int q = 0; q < V; ++q) Ek1[c][q] = S(0);
-    if (lact && more && k + 2 < g.Nz) {
-      const I n2 = col + sz * (I)(k + 2);
-      ldv<V>(Ein, n2, Ek1[0]); ldv<V>(Ein, N + n2, Ek1[1]); ldv<V>(Ein, 2 * N + n2, Ek1[2]);
+        for (int q = 0; q < V; ++q) e0(c, P, q) = Ek1[c][q];
     }
-    if (lact && own && l2e) {
-      S c1yp[V];
-      ldsv(sCy(p, 1) + xi, c1yp);
-      S HX[V + 1], HY[V + 1], HZ[V + 1];
-#pragma unroll
-      for (int q = 0; q < V + 1; ++q) {
-        HX[q] = sH2(0, w - 1)[atx(q - 1)];
-        HY[q] = sH2(1, w - 1)[atx(q - 1)];
-        HZ[q] = sH2(2, w - 1)[atx(q - 1)];
-      }
-      const I np = col + sz * (I)p;
-      S E2[3][V], Jn[3][V];
+    const int kn = k < kend ? k + 1 : g.Nz;  // nothing is read after the last plane
+    Row row;
+    load_row(kn, row);
+    const uint32_t coden = load_code(kn);
+    load_e(k < kend ? k + 2 : g.Nz, Ek1);
+    if (own && l2e) {
+      const S itaxp = rowv(1, rp), tLzp = plv(1, p), bv2 = plv(3, p);
+      S c1yp[V], tLx[V];
+      ldsv(cyv(1, rp), c1yp);
+      ldsv(sX + (Q + ln) * V, tLx);
+      const S HYm = h2(1, Pd - 1, V - 1), HZm = h2(2, Pd - 1, V - 1);
+      S E2[3][V], s2[V], Jn[3][V];
 #pragma unroll
       for (int q = 0; q < V; ++q) {
         const S *t = sMat + NM * (int)((codep >> (8 * q)) & 0xffu);
-        const S b0 = (S)(t[3] * itaxp), b1 = (S)(t[4] * c1yp[q]), b2 = (S)(t[5] * itAz[q]);
-        S d0 = e_sum<S>(b0, tLy, tLzp, H2p[1][q], HY[q + 1], sH2(2, w - 2)[atx(q)],
-                        HZ[q + 1], +1, -1);
-        S d1 = e_sum<S>(b1, tLx[q], tLzp, H2p[0][q], HX[q + 1], HZ[q], HZ[q + 1], -1, +1);
-        S d2 = e_sum<S>(b2, tLx[q], tLy, sH2(0, w - 2)[atx(q)], HX[q + 1], HY[q],
-                        HY[q + 1], +1, -1);
-        const S e0 = sE1(0, w - 1)[atx(q)], e1 = sE1(1, w - 1)[atx(q)];
-        const S e2 = sE1(2, w - 1)[atx(q)];  // E1(k-1)
+        const S b0 = (S)(t[3] * itaxp), b1 = (S)(t[4] * c1yp[q]), b2 = (S)(t[5] * itAz[0][q]);
+        S d0 = e_sum<S>(b0, tLy, tLzp, H2p[1][q], H2[1][q], h2(2, Pdd, q), H2[2][q], +1, -1);
+        S d1 = e_sum<S>(b1, tLx[q], tLzp, H2p[0][q], H2[0][q], q ? H2[2][q - 1] : HZm, H2[2][q],
+                        -1, +1);
+        S d2 = e_sum<S>(b2, tLx[q], tLy, h2(0, Pdd, q), H2[0][q], q ? H2[1][q - 1] : HYm,
+                        H2[1][q], +1, -1);
+        s2[q] = d2;
+        const S o0 = e1(0, Pd, q), o1 = e1(1, Pd, q), o2 = e1(2, Pd, q);  // E1(k-1)
         if (COND) {
-          d0 = d0 - t[3] * (S)(t[6] * e0);
-          d1 = d1 - t[4] * (S)(t[7] * e1);
-          d2 = d2 - t[5] * ((q == qbeam) ? bv2 : (S)(t[8] * e2));
-        } else if (q == qbeam) {
-          d2 = d2 - t[5] * bv2;
+          d0 = d0 - t[3] * (S)(t[6] * o0);
+          d1 = d1 - t[4] * (S)(t[7] * o1);
+          d2 = d2 - t[5] * (S)(t[8] * o2);
         }
-        E2[0][q] = (S)(e0 + dt * d0);
-        E2[1][q] = (S)(e1 + dt * d1);
-        E2[2][q] = (S)(e2 + dt * d2);
-        if (!COND && q == qbeam) *atw(J, 2 * N + np + (I)q) = bv2;
-        if (COND && !x.skip_j) {  // J = sigma E2 by the call's last launch
+        E2[0][q] = (S)(o0 + dt * d0);
+        E2[1][q] = (S)(o1 + dt * d1);
+        E2[2][q] = (S)(o2 + dt * d2);
+      }
+      if (qbeam >= 0) {
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+          const S *t = sMat + NM * (int)((codep >> (8 * q)) & 0xffu);
+          const S d2 = s2[q] - t[5] * bv2;
+          if (q == qbeam) E2[2][q] = (S)(e1(2, Pd, q) + dt * d2);
+        }
+        if (!COND) J[2 * g.N + (int64_t)p * g.sz + cell + qbeam] = bv2;
+      }
+      if (capq0 < capq1 && x.cap_sample + 1 < x.cap_samples) capture(g.Nz + p, E2[2]);
+      buf_st<RAG>(bEo, ofs, (I)p * sz * ES, NB, E2);
+      if (COND && !x.skip_j) {  // J = sigma E2 by the call's last launch
+        const Buf bJ = buf_of(J, 3 * NB);
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+          const S *t = sMat + NM * (int)((codep >> (8 * q)) & 0xffu);
 #pragma unroll
           for (int c = 0; c < 3; ++c) Jn[c][q] = (S)(t[6 + c] * E2[c][q]);
         }
-        if (cap2 && q >= capq0 && q < capq1)
-          cap[capb2 + (int64_t)(q + xi - x.cap_ix0) * capl + p] = E2[2][q];
-      }
-      stv_nt<V>(Eout, np, E2[0]); stv_nt<V>(Eout, N + np, E2[1]);
-      stv_nt<V>(Eout, 2 * N + np, E2[2]);
-      if (COND && !x.skip_j) {
-        stv_nt<V>(J, np, Jn[0]); stv_nt<V>(J, N + np, Jn[1]); stv_nt<V>(J, 2 * N + np, Jn[2]);
+        buf_st<RAG>(bJ, ofs, (I)p * sz * ES, NB, Jn);
       }
     }
 #pragma unroll
-    for (int q = 0; q < V; ++q) { H2p[0][q] = H2c[0][q]; H2p[1][q] = H2c[1][q]; }
+    for (int q = 0; q < V; ++q) { H2p[0][q] = H2[0][q]; H2p[1][q] = H2[1][q]; }
     if (doE1) {
 #pragma unroll
       for (int c = 0; c < 3; ++c)
 #pragma unroll
-        for (int q = 0; q < V; ++q) sE1(c, w - 1)[atx(q)] = E1[c][q];
+        for (int q = 0; q < V; ++q) e1(c, Pd, q) = E1[c][q];
     }
-    put_ring(k + 1, P);
-    load_plane_b(more ? k + 1 : g.Nz, P);
+    put_row(k + 1, row);
+    load_h(kn, h0);
     // level 2 of the next plane uses this plane's coefficients
     codep = code;
+    code = coden;
     __syncthreads();
   }
+}
+
+template <typename S, bool COND, bool DESC, bool RAG>
+__global__ void __launch_bounds__(T2_NT)
+k_fused4_t2(GridDev g, MetricDev<S> m, const S *__restrict__ Ein, const S *__restrict__ Hin,
+            S *__restrict__ Eout, S *__restrict__ Hout, S *__restrict__ J, Coefs<S> cf, S dt,
+            T2Aux x, const S *__restrict__ beam1, const S *__restrict__ beam2,
+            S *__restrict__ cap) {
+  t2_tile<S, COND, DESC, RAG>(g, m, Ein, Hin, Eout, Hout, J, cf, dt, x, beam1, beam2, cap,
+                             xcd_tile(blockIdx.x, x.ntx * x.nty * x.ntz));
 }
 
 }  // namespace wf

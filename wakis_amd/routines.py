@@ -100,8 +100,9 @@ class RoutinesMixin:
         the same way, and the result is bitwise that of the uninterrupted run.
         The fields are checked for Inf/NaN on the device at the end
         (``fields_finite``). Runs of 2,000 steps or more on grids of 2^22
-        cells or more first time the fused kernel's workgroup shapes
-        (``tune_fused``); the fields are bitwise the same for every shape.
+        cells or more that do not take two steps per launch first time the
+        fused kernel's workgroup shapes (``tune_fused``); the fields are
+        bitwise the same for every shape.
         """
         if wake is not None:
             self.wake = wake
@@ -117,8 +118,15 @@ class RoutinesMixin:
                                  "and a checkpoint file name")
         ctx = self._wake_setup(wakelength, compute_plane)
         Nt = ctx["Nt"]
-        if Nt >= 2000 and self.N >= (1 << 22):  # long run: measure the kernel shapes first
-            self.tune_fused(lambda k: self._wake_args(ctx, 0, k))
+        if Nt >= 2000 and self.N >= (1 << 22):
+            # long run: measure the kernel shapes first, unless it takes two steps
+            # per launch, which no shape of one step per launch beats (the trials
+            # took 44 of 712 ms of a 3,600-step run at 256x256x512)
+            mon = use_field_monitor and field_monitor is not None
+            per_call = min(1 if callback is not None else Nt if chunk is None else int(chunk),
+                           Nt if every is None else every)
+            if mon or per_call < 3 or not self._pairs_apply(self._wake_args(ctx, 0, 3)):
+                self.tune_fused(lambda k: self._wake_args(ctx, 0, k))
         if save_J:  # J_z on the window before the run, for Jz.h5
             ix0, iy0, nx, ny = ctx["win"]
             ctx["J0"] = self.J.to_matrix("z")[ix0:ix0 + nx, iy0:iy0 + ny, :].reshape(

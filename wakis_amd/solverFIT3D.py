@@ -194,9 +194,8 @@ class SolverFIT3D(RoutinesMixin):
         # sets -1 = segments or N), -1 row segments
         self.fused_full_rows = 0
         # two leapfrog steps per launch where that kernel applies (the wakefield
-        # step with material codes, FP32 or FP64, Nx <= 256): 0 off, 1 on (8 rows
-        # per workgroup, FP64 2), 4 or 8 rows (FP32); bit-identical to one step
-        # per launch.
+        # step with material codes): 0 off, 1 on, 4 or 8: at most so many rows
+        # per workgroup; bit-identical to one step per launch.
         # tune_fused() sets 0 when one step per launch measures faster
         self.fused_two_step = 1
         # {full_rows: ms per step} of the last tune_fused(); -2: two steps per launch
@@ -221,7 +220,8 @@ class SolverFIT3D(RoutinesMixin):
         self._J_clean_version = self.J.version
         self._sigmaE_versions = (self.E.version, self.J.version)  # J == sigma*E (all zero)
         self.last_path = None
-        self.last_two_step = False  # the last step call ran two steps per launch
+        self.last_two_step = False  # the last step call ran two steps per launch to its end
+        self.last_pairs = False  # it ran two steps per launch, the end perhaps one at a time
         self.solverInitializationTime = time.time() - t0
         # the reference's solver log keys (solverFIT3D.py:149, 171-176, 234, 281, 299, 350-354)
         self.update_logger(["use_gpu", "use_mpi", "grid", "background", "bc_low", "bc_high"])
@@ -777,9 +777,22 @@ class SolverFIT3D(RoutinesMixin):
         _lib.check(_lib.lib().wf_step(self._handle, ctypes.byref(args), _lib.stream_ptr()),
                    "wf_step")
         # two steps per launch with an even count: the last launch was a pair
-        self.last_two_step = bool(args.two_step_used)
+        self.last_two_step = args.two_step_used == 1
+        self.last_pairs = args.two_step_used != 0
         self._finish_run(fused, bool(args.result_swapped), keep,
                          pair_last=self.last_two_step and args.nsteps % 2 == 0)
+
+    def _pairs_apply(self, args):
+        """Whether a long call with these arguments runs two steps per launch
+        (the rule of the library, lib_fused_t2.hip)."""
+        if not self._prepare_fused(args):
+            return False
+        size = np.dtype(self.dtype).itemsize
+        box = all(h > l for l, h in zip(args.box_lo, args.box_hi))
+        return bool(args.two_step and args.code and args.zero_masked and not args.code_escape
+                    and args.beam_table and 3 * self.N * size < 2 ** 32 and args.variant == 0
+                    and args.full_rows <= 0 and args.cells_per_lane in (0, 16 // size)
+                    and not box and not args.traj_E and not args.mon_acc)
 
     def tune_fused(self, make_args=None, steps=3):
         """Choose the fused kernel's workgroup shape by timing it (no reference
@@ -799,13 +812,22 @@ class SolverFIT3D(RoutinesMixin):
                 or self.path == "general"):
             return None
         make = make_args if make_args is not None else self._step_args
-        if not self._choose_fused(make(steps)):
+        args = make(steps)
+        if not self._choose_fused(args):
             return None
+        size = np.dtype(self.dtype).itemsize
+        if self._pairs_apply(args) and (self.Nx > 256 or self.Nx % (16 // size) != 0
+                                        or self.fused_two_step == 1 and (
+                                            self.N < 1 << 20 or size == 8 and self.Nx < 224)):
+            # calls that end with single steps: a trial of a few steps times
+            # those, and no shape of one step per launch beat pairs of steps
+            # where measured (row segments or whole rows, 17 grids)
+            self.fused_full_rows, self.fused_tuning = -1, {}
+            return -1
         # with two steps per launch, warm up and time whole launches (even counts)
         warm = 2 if self.fused_two_step else 1
         if self.fused_two_step:
             steps += steps % 2
-        size = np.dtype(self.dtype).itemsize
         vn = 16 // size
         if self.Nx % vn:
             return None
