@@ -383,8 +383,10 @@ int wf_wake_wp(const void *capture, int32_t dtype, int32_t nlines, int64_t cap_s
   if (dtype != WF_F64 && dtype != WF_F32) return fail(WF_EINVAL, "wf_wake_wp: bad dtype");
   if (ns == 0) return WF_OK;
   hipStream_t st = (hipStream_t)stream;
+  const size_t lds = nz <= wf::WP_COLS_MAX ? (size_t)nz * wf::WP_NS * sizeof(int) : 0;
 #define WF_WP_LAUNCH(S, CM)                                                                   \
-  hipLaunchKernelGGL((wf::k_wake_wp<S, CM>), dim3(nblocks(ns, 256)), dim3(256), 0, st,        \
+  hipLaunchKernelGGL((wf::k_wake_wp<S, CM>), dim3(nblocks(ns, wf::WP_NS)),                    \
+                     dim3(wf::WP_THREADS), lds, st,                                           \
                      (const S *)capture, nlines, cap_samples, Nz, k0, nz, z, dz, s, ns, v,    \
                      zref_v, t0, ti, dt, nt, ncols, qe12, WP3d)
   if (dtype == WF_F64) {
@@ -404,8 +406,9 @@ int wf_wake_trans(const double *WP3d, int64_t ns, double ds, double dxsum, doubl
   if (!WP3d || !WPx || !WPy) return fail(WF_EINVAL, "wf_wake_trans: null argument");
   if (ns < 0) return fail(WF_ERANGE, "wf_wake_trans: ns < 0");
   if (ns == 0) return WF_OK;
-  hipLaunchKernelGGL(wf::k_wake_trans, dim3(nblocks(ns, 256)), dim3(256), 0, (hipStream_t)stream,
-                     WP3d, ns, ds, dxsum, dysum, WPx, WPy);
+  if (ns > 2147483647LL) return fail(WF_ERANGE, "wf_wake_trans: ns too large");
+  hipLaunchKernelGGL(wf::k_wake_trans, dim3((unsigned)ns), dim3(256), 0, (hipStream_t)stream, WP3d,
+                     ns, ds, dxsum, dysum, WPx, WPy);
   WF_LAUNCH_CHECK();
   return WF_OK;
 }
@@ -417,9 +420,19 @@ int wf_dft(const double *x, int32_t nsig, int64_t len, int64_t N, int64_t nbins,
     return fail(WF_ERANGE, "wf_dft: inconsistent sizes");
   if (nbins == 0) return WF_OK;
   if (nbins > 2147483647LL || nsig > 65535) return fail(WF_ERANGE, "wf_dft: too many bins");
-  hipLaunchKernelGGL(wf::k_dft, dim3((unsigned)nbins, (unsigned)nsig), dim3(256), 0,
-                     (hipStream_t)stream, x, len, N, nbins, out);
-  WF_LAUNCH_CHECK();
+  hipStream_t st = (hipStream_t)stream;
+  for (int sig = 0; sig < nsig; sig += 4) {  // up to four signals per launch
+    const double *xs = x + (int64_t)sig * len;
+    double *os = out + (int64_t)sig * nbins * 2;
+    const dim3 grd((unsigned)nbins), blk(256);
+    switch (std::min(nsig - sig, 4)) {
+      case 1: hipLaunchKernelGGL(wf::k_dft<1>, grd, blk, 0, st, xs, len, N, nbins, os); break;
+      case 2: hipLaunchKernelGGL(wf::k_dft<2>, grd, blk, 0, st, xs, len, N, nbins, os); break;
+      case 3: hipLaunchKernelGGL(wf::k_dft<3>, grd, blk, 0, st, xs, len, N, nbins, os); break;
+      default: hipLaunchKernelGGL(wf::k_dft<4>, grd, blk, 0, st, xs, len, N, nbins, os); break;
+    }
+    WF_LAUNCH_CHECK();
+  }
   return WF_OK;
 }
 
