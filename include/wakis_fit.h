@@ -318,7 +318,10 @@ int wf_count_nonfinite_noalloc(const void *x, int32_t dtype, int64_t n, int32_t 
  * step covers the tiles of every grid (3 rows per workgroup, cells_per_lane 1
  * or the 16-byte width, 0 = 16-byte width; kz z-planes per workgroup, 0 = 32).
  * Even steps read E/H and write E2/H2, odd steps the reverse: after steps
- * [0, S) grid i's fields are in E2/H2 iff min(S, nsteps_i) is odd. Results are
+ * [0, S) grid i's fields are in E2/H2 iff min(S, nsteps_i) is odd. With kz 0, row
+ * segments, material codes, beam tables, no trajectories and two_step != 0 on
+ * every item, launches advance the grids by two steps where four and one more
+ * are left (cells_per_lane is then the tile of the single steps). Results are
  * bit-identical to wf_step on each grid. wf_batch_create copies the
  * descriptors to the device (the only allocation); the batch must not outlive
  * the handles and buffers it names. */

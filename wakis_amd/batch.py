@@ -85,8 +85,9 @@ def wakesolve_batch(solvers, wakelength, compute_plane="both", cells_per_lane=No
     (coefficient arrays, masks applied in the kernel); otherwise
     BatchNotApplicable is raised before anything runs. ``cells_per_lane``/``kz``/
     ``full_rows`` (whole-row workgroups, rows per grid picked) fix the tile shape; with
-    ``autotune`` the candidates are timed on successive chunks of
-    ``tune_steps`` steps of the run itself and the fastest runs the rest.
+    ``autotune`` grids on material codes take two steps per launch, others time
+    the candidates on successive chunks of ``tune_steps`` steps of the run
+    itself and the fastest runs the rest.
     Returns a dict with the chosen shape, the step count and the timing.
     """
     if not solvers:
@@ -108,8 +109,15 @@ def wakesolve_batch(solvers, wakelength, compute_plane="both", cells_per_lane=No
     if len({bool(a.code) for a in args}) != 1:
         raise BatchNotApplicable("all grids of a batch use material codes, or none")
     nmax = max(ctx["Nt"] for ctx in ctxs)
+    nat = _native_width(solvers[0].dtype)
     if cells_per_lane is not None or kz is not None or full_rows is not None or not autotune:
         cands = [(cells_per_lane or 0, kz or 0, bool(full_rows))]
+        for a in args:  # the caller's tile shape: one step per launch
+            a.two_step = 0
+    elif all(s._pairs_apply(a, prepared=True) for s, a in zip(solvers, args)):
+        # two steps per launch in the library's tiles: nothing to try (the six
+        # shapes of one step per launch took a quarter of a 600-step run of 24 grids)
+        cands = [(nat if all(s.Nx % nat == 0 for s in solvers) else 1, 0, False)]
     else:
         cands = _candidates(solvers)
     ev0 = torch.cuda.Event(enable_timing=True)

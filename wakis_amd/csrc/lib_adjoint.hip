@@ -330,7 +330,7 @@ int batch_adj_build(wf_handle *const *hs, const wf_adjoint_args *as, const int32
   WF_HIP(hipMalloc(&b->desc_dev, sizeof(wf::AdjBatchDesc<S, A>) * n));
   WF_HIP(hipMemcpy(b->desc_dev, d.data(), sizeof(wf::AdjBatchDesc<S, A>) * n,
                    hipMemcpyHostToDevice));
-  WF_HIP(hipMalloc((void **)&b->step_dev, sizeof(int)));
+  WF_HIP(hipMalloc((void **)&b->step_dev, 3 * sizeof(int)));
   return WF_OK;
 }
 
@@ -411,7 +411,7 @@ int wf_batch_adjoint_run(wf_batch_adjoint *b, int32_t r0, int32_t nr, int32_t us
   if (!b) return fail(WF_EINVAL, "wf_batch_adjoint_run: null batch");
   if (r0 < 0 || nr < 0) return fail(WF_EINVAL, "wf_batch_adjoint_run: negative step range");
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(wf::k_batch_set, dim3(1), dim3(1), 0, st, b->step_dev, (int)r0);
+  hipLaunchKernelGGL(wf::k_batch_set, dim3(1), dim3(1), 0, st, b->step_dev, (int)r0, 0, 0);
   WF_LAUNCH_CHECK();
   int done = 0;
   if (use_graph && nr >= BATCH_GRAPH_STEPS) {

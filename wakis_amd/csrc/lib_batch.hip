@@ -10,7 +10,10 @@ struct wf_batch {
   int fr = 0;                 // whole-row tiles (16-byte lanes), rows per grid
   size_t lds = 0;
   void *desc_dev = nullptr;   // BatchDesc<S>[ninst]
-  int *step_dev = nullptr;    // step number read by the batch kernel
+  int *step_dev = nullptr;    // step number read by the batch kernel, the run's range
+  int pairs = 0;              // steps taken in pairs where a grid has four left and one more
+  batch_t2 t2;
+  std::vector<int> nsteps;
   hipStream_t cap_stream = nullptr;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
@@ -82,6 +85,7 @@ int batch_build(wf_handle *const *hs, const wf_step_args *as, int n, int vw, int
     e.cap = a->capture ? (S *)a->capture : nullptr;
     e.cap_sample0 = a->cap_sample0;
     e.nsteps = a->nsteps;
+    e.pairs = 0;
     e.tile0 = (int)tiles;
     tiles += (int64_t)x.ntx * x.nty * x.ntz;
     e.thr0 = b->traj_threads;
@@ -98,9 +102,15 @@ int batch_build(wf_handle *const *hs, const wf_step_args *as, int n, int vw, int
   if (tiles > 2147483647LL) return fail(WF_ERANGE, "wf_batch_create: too many tiles");
   b->ntiles = (int)tiles;
   b->lds = lds;
+  if (b->pairs) {
+    const int rc = batch_t2_build(b->dtype, d.data(), hs, as, n, &b->t2);
+    if (rc < 0) return rc;
+    b->pairs = rc;
+    for (auto &e : d) e.pairs = rc;
+  }
   WF_HIP(hipMalloc(&b->desc_dev, sizeof(wf::BatchDesc<S>) * n));
   WF_HIP(hipMemcpy(b->desc_dev, d.data(), sizeof(wf::BatchDesc<S>) * n, hipMemcpyHostToDevice));
-  WF_HIP(hipMalloc((void **)&b->step_dev, sizeof(int)));
+  WF_HIP(hipMalloc((void **)&b->step_dev, 3 * sizeof(int)));
   return WF_OK;
 }
 
@@ -161,6 +171,41 @@ int batch_step_once(const wf_batch *b, hipStream_t st) {
   return b->dtype == WF_F64 ? batch_launch<double>(b, st) : batch_launch<float>(b, st);
 }
 
+// Steps [step0, step0 + nsteps) with pairs: by fours, two pair launches over the
+// grids that take these four in pairs, and single steps over the others.
+int batch_run_pairs(const wf_batch *b, int step0, int nsteps, hipStream_t st) {
+  const int end = step0 + nsteps;
+  for (int s = step0; s < end; s += 4) {
+    bool two = false;
+    int one0 = end, one1 = s;  // single steps of these four
+    for (const int ns : b->nsteps) {
+      const int s0 = wf::batch_single0(ns, step0, end, 1);
+      two = two || s0 > s;
+      const int lo = std::max(s0, s), hi = std::min(std::min(ns, s + 4), end);
+      if (lo < hi) {
+        one0 = std::min(one0, lo);
+        one1 = std::max(one1, hi);
+      }
+    }
+    if (two) {
+      for (int p = 0; p < 2; ++p) {
+        const int rc = batch_t2_launch(b->dtype, &b->t2, b->ninst, b->cond, b->desc, s + 2 * p,
+                                       step0, end, (s & 1) ^ p, st);
+        if (rc != WF_OK) return rc;
+      }
+    }
+    if (one0 < one1) {
+      hipLaunchKernelGGL(wf::k_batch_set, dim3(1), dim3(1), 0, st, b->step_dev, one0, step0, end);
+      WF_LAUNCH_CHECK();
+      for (int t = one0; t < one1; ++t) {
+        const int rc = batch_step_once(b, st);
+        if (rc != WF_OK) return rc;
+      }
+    }
+  }
+  return WF_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -215,6 +260,16 @@ int wf_batch_create(wf_handle *const *handles, const wf_step_args *args, int32_t
   b->cond = a0.conductive; b->jm = a0.jmode; b->desc = h0->g.m1desc;
   b->lut = (a0.code && a0.mat && a0.nmat > 0 && a0.metric2d) ? 1 : 0;
   b->fr = fr;
+  // the wakefield step of every grid, as for a single grid (fused_t2_applies), and
+  // the tile shape left to the library
+  b->pairs = (b->lut && !fr && kz == 0) ? 1 : 0;
+  for (int i = 0; i < n; ++i) {
+    const wf_step_args *a = &args[i];
+    b->nsteps.push_back(a->nsteps);
+    if (!a->two_step || !a->beam_table || a->traj_E ||
+        a->jmode != (a->conductive ? WF_J_FULL : WF_J_LINE))
+      b->pairs = 0;
+  }
   const int rc = dtype == WF_F64 ? batch_build<double>(handles, args, n, vw, kz, b)
                                  : batch_build<float>(handles, args, n, vw, kz, b);
   if (rc != WF_OK) {
@@ -229,7 +284,8 @@ int wf_batch_run(wf_batch *b, int32_t step0, int32_t nsteps, int32_t use_graph, 
   if (!b) return fail(WF_EINVAL, "wf_batch_run: null batch");
   if (step0 < 0 || nsteps < 0) return fail(WF_EINVAL, "wf_batch_run: negative step range");
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(wf::k_batch_set, dim3(1), dim3(1), 0, st, b->step_dev, (int)step0);
+  if (b->pairs) return batch_run_pairs(b, step0, nsteps, st);
+  hipLaunchKernelGGL(wf::k_batch_set, dim3(1), dim3(1), 0, st, b->step_dev, (int)step0, 0, 0);
   WF_LAUNCH_CHECK();
   int done = 0;
   if (use_graph && nsteps >= BATCH_GRAPH_STEPS) {
@@ -263,6 +319,7 @@ int wf_batch_destroy(wf_batch *b) {
   if (b->cap_stream) hipStreamDestroy(b->cap_stream);
   if (b->desc_dev) hipFree(b->desc_dev);
   if (b->step_dev) hipFree(b->step_dev);
+  if (b->t2.desc_dev) hipFree(b->t2.desc_dev);
   delete b;
   return WF_OK;
 }

@@ -48,8 +48,10 @@ constexpr size_t t2_static_lds() {
 // the time of a plane. Fitted to 9 to 120 shapes of each of 17 grids from
 // 32x32x64 to 333x300x100 (FP32, FP64, with and without conduction): the shape
 // it picks is within 2% of the best measured one on average, 9% at most.
+// `others`: workgroups of other grids on the machine beside these.
 template <typename S>
-T2Shape t2_shape(const wf::GridDev &g, int nmat, int ncu, int want_rows, int want_kz) {
+T2Shape t2_shape(const wf::GridDev &g, int nmat, int ncu, int want_rows, int want_kz,
+                 int others = 0) {
   constexpr int V = 16 / (int)sizeof(S);
   using C = wf::T2Slots;
   T2Shape out;
@@ -95,7 +97,7 @@ T2Shape t2_shape(const wf::GridDev &g, int nmat, int ncu, int want_rows, int wan
         const double w = (4 * s.T + 6) * Q / 64.0 + (Q % 64 ? 4 : 0);
         const double lines = std::ceil(s.ln / 8.0) + (ntx > 1 || g.Nx * sizeof(S) % 128 ? 1 : 0);
         const double bytes = 6 * ((s.T + 3.5) * lines * 128 + s.T * s.ln * 16.0);
-        const double busy = (double)std::min<int64_t>(wgs, ncu);
+        const double busy = (double)std::min<int64_t>(wgs, ncu) + others;
         const double plane = std::max(std::max(0.12 * w, bytes * busy / 6.5e6), 3.0);
         const double t = (double)rounds * (s.KZ + 3) * plane;
         if (t < best * 0.999) { best = t; out = s; }
@@ -103,6 +105,17 @@ T2Shape t2_shape(const wf::GridDev &g, int nmat, int ncu, int want_rows, int wan
     }
   }
   return out;
+}
+
+inline void t2_aux(const T2Shape &sh, const wf::GridDev &g, const wf_step_args *a, wf::T2Aux &x) {
+  x.ixs = a->ixs;
+  x.iys = a->iys;
+  x.cap_ix0 = a->cap_ix0; x.cap_iy0 = a->cap_iy0; x.cap_nx = a->cap_nx; x.cap_ny = a->cap_ny;
+  x.cap_samples = a->cap_samples;
+  x.ntx = sh.ntx; x.T = sh.T; x.OW = sh.OW; x.Q = sh.Q; x.QS = sh.QS;
+  x.l0 = sh.l0; x.ln = sh.ln; x.KZ = sh.KZ;
+  x.nty = (g.Ny + sh.T - 1) / sh.T;
+  x.ntz = (g.Nz + sh.KZ - 1) / sh.KZ;
 }
 
 template <typename S>
@@ -116,14 +129,7 @@ int launch_t2(wf_handle *h, wf_step_args *a, const wf::MetricDev<S> &m, hipStrea
     return sizeof(S) == 4 ? step_fused_f32(h, a, st) : step_fused_f64(h, a, st);
   }
   wf::T2Aux x{};
-  x.ixs = a->ixs;
-  x.iys = a->iys;
-  x.cap_ix0 = a->cap_ix0; x.cap_iy0 = a->cap_iy0; x.cap_nx = a->cap_nx; x.cap_ny = a->cap_ny;
-  x.cap_samples = a->cap_samples;
-  x.ntx = sh.ntx; x.T = sh.T; x.OW = sh.OW; x.Q = sh.Q; x.QS = sh.QS;
-  x.l0 = sh.l0; x.ln = sh.ln; x.KZ = sh.KZ;
-  x.nty = (g.Ny + sh.T - 1) / sh.T;
-  x.ntz = (g.Nz + sh.KZ - 1) / sh.KZ;
+  t2_aux(sh, g, a, x);
   const bool rag = g.Nx % V != 0, cond = a->conductive != 0, desc = g.m1desc != 0;
   const T2Fn<S> kern = pick_t2<S>(cond, desc, rag);
   const int threads = ((sh.T + 4) * sh.Q + 63) / 64 * 64;

@@ -109,6 +109,9 @@ constexpr int FR_BOUND = 7;            // full-row kernels: up to 64 * 8 threads
 constexpr size_t FR_LDS_MAX = 65536;   // and 64 KiB of LDS per workgroup
 
 constexpr int BATCH_GRAPH_STEPS = 16;  // batch steps captured in one HIP graph
+// workgroups per CU of a batch's pair launch (24 grids of 28 to 160 cells a side:
+// 1.5 and 2 took 9% longer, the halo planes of the shorter chunks)
+constexpr double BATCH_T2_LOAD = 1.0;
 
 // Argument checks shared by wf_step and wf_batch_create.
 WF_HIDDEN const char *check_traj(const wf_handle *h, const void *tE, const void *tH,
@@ -129,3 +132,16 @@ WF_HIDDEN int step_fused_t2_f32(wf_handle *h, wf_step_args *a, hipStream_t st,
 WF_HIDDEN int step_fused_t2_f64(wf_handle *h, wf_step_args *a, hipStream_t st,
                                 bool end_paired);
 WF_HIDDEN int step_fused_f64(wf_handle *h, wf_step_args *a, hipStream_t st);
+
+// Pairs of steps of a batch (lib_batch_t2.hip): descriptors and launch shape.
+struct batch_t2 {
+  void *desc_dev = nullptr;  // T2Batch<S>[n]
+  int ntiles = 0, threads = 0, rag = 0;
+  size_t lds = 0;
+};
+// 1 built, 0 no tile fits a grid (one step per launch then), < 0 an error
+WF_HIDDEN int batch_t2_build(int dtype, const void *batch_desc, wf_handle *const *hs,
+                             const wf_step_args *as, int n, batch_t2 *t);
+// steps s, s + 1 of a run of [step0, end); flip: the launch reads E2/H2
+WF_HIDDEN int batch_t2_launch(int dtype, const batch_t2 *t, int n, int cond, int desc, int s,
+                              int step0, int end, int flip, hipStream_t st);

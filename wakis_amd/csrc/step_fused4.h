@@ -609,6 +609,7 @@ struct BatchDesc {
   S *cap;
   int64_t cap_sample0;         // capture sample written by step s: cap_sample0 + s
   int nsteps;                  // the grid takes part in steps 0 .. nsteps-1
+  int pairs;                   // its steps before batch_single0 are taken in pairs
   int tile0;                   // its first tile in the batch's tile numbering
   // optional region trajectory (reverse mode): after step s, slot traj_slot0+s+1
   S *tE, *tH;                  // [slots][3 * box cells], or null
@@ -616,6 +617,16 @@ struct BatchDesc {
   int64_t traj_slot0;
   int64_t thr0;                // first thread of this grid in the batched gather
 };
+
+// First step that a grid of nsteps steps takes singly in a run of the steps
+// [step0, end): the steps before it are taken in twos of pairs (four steps and
+// two exchanges of the buffers, so that even steps still read E/H), and the
+// grid's last step is always single (the spare buffers then hold the fields one
+// step back, and J is stored).
+__host__ __device__ inline int batch_single0(int nsteps, int step0, int end, int pairs) {
+  const int lim = end >= nsteps ? nsteps - 1 : end;
+  return (pairs && lim > step0) ? step0 + (lim - step0) / 4 * 4 : step0;
+}
 
 // One step of every grid of a batch in one launch. The step number comes from
 // device memory (k_batch_next advances it), so a captured graph of these
@@ -635,7 +646,9 @@ k_fused4_batch(const BatchDesc<S> *__restrict__ d, int ninst, int ntiles,
     else hi = mid - 1;
   }
   const BatchDesc<S> &b = d[lo];
-  if (step >= b.nsteps) return;  // whole workgroup, before any barrier
+  // whole workgroup, before any barrier (step_ptr[1], [2]: the run's range)
+  if (step >= b.nsteps) return;
+  if (b.pairs && step < batch_single0(b.nsteps, step_ptr[1], step_ptr[2], 1)) return;
   const bool odd = step & 1;
   FusedAux x = b.x;
   x.cap_sample = b.cap_sample0 + step;
@@ -647,6 +660,10 @@ k_fused4_batch(const BatchDesc<S> *__restrict__ d, int ninst, int ntiles,
 }
 
 static __global__ void k_batch_next(int *step) { step[0] = step[0] + 1; }
-static __global__ void k_batch_set(int *step, int v) { step[0] = v; }
+static __global__ void k_batch_set(int *step, int v, int step0, int end) {
+  step[0] = v;
+  step[1] = step0;
+  step[2] = end;
+}
 
 }  // namespace wf

@@ -583,4 +583,42 @@ k_fused4_t2(GridDev g, MetricDev<S> m, const S *__restrict__ Ein, const S *__res
                              xcd_tile(blockIdx.x, x.ntx * x.nty * x.ntz));
 }
 
+// One grid of a batch that takes its steps in pairs (BatchDesc) and its tiles.
+template <typename S>
+struct T2Batch {
+  BatchDesc<S> b;
+  T2Aux x;    // cap_sample is set per launch
+  int tile0;  // its first tile in the numbering of the pair launches
+};
+
+// Steps s and s + 1 of every grid that takes both in a pair, in one launch. The
+// run covers the steps [step0, end); `flip`: the launch reads E2/H2. Each grid has
+// its share of the CUs, one workgroup each. 24 grids of 28 to 160 cells a side
+// (5.3 million cells), FP32: about 100 us per launch, 50 a step, against 92 + 4.5
+// of the one-step kernel and its step counter.
+template <typename S, bool COND, bool DESC, bool RAG>
+__global__ void __launch_bounds__(T2_NT)
+k_fused4_t2_batch(const T2Batch<S> *__restrict__ d, int ninst, int ntiles, int s, int step0,
+                  int end, int flip) {
+  const int tile = xcd_tile(blockIdx.x, ntiles);
+  int lo = 0, hi = ninst - 1;  // last descriptor with tile0 <= tile
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (d[mid].tile0 <= tile) lo = mid;
+    else hi = mid - 1;
+  }
+  const T2Batch<S> &e = d[lo];
+  if (s >= batch_single0(e.b.nsteps, step0, end, 1)) return;  // whole workgroup
+  T2Aux x = e.x;
+  x.cap_sample = e.b.cap_sample0 + s;
+  x.skip_j = 1;  // J is stored by the single steps at a grid's end
+  const GridDev g = e.b.g;
+  const MetricDev<S> m = e.b.m;
+  const Coefs<S> cf = e.b.cf;
+  const S *row = e.b.beam_table + (e.b.beam_row0 + s) * g.Nz;
+  t2_tile<S, COND, DESC, RAG>(g, m, flip ? e.b.E2 : e.b.E, flip ? e.b.H2 : e.b.H,
+                              flip ? e.b.E : e.b.E2, flip ? e.b.H : e.b.H2, e.b.J, cf, e.b.dt, x,
+                              row, row + g.Nz, e.b.cap, tile - e.tile0);
+}
+
 }  // namespace wf

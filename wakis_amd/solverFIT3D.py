@@ -782,10 +782,11 @@ class SolverFIT3D(RoutinesMixin):
         self._finish_run(fused, bool(args.result_swapped), keep,
                          pair_last=self.last_two_step and args.nsteps % 2 == 0)
 
-    def _pairs_apply(self, args):
+    def _pairs_apply(self, args, prepared=False):
         """Whether a long call with these arguments runs two steps per launch
-        (the rule of the library, lib_fused_t2.hip)."""
-        if not self._prepare_fused(args):
+        (the rule of the library, lib_fused_t2.hip). ``prepared``: the
+        arguments have been through ``_prepare_fused``."""
+        if not prepared and not self._prepare_fused(args):
             return False
         size = np.dtype(self.dtype).itemsize
         box = all(h > l for l, h in zip(args.box_lo, args.box_hi))
