@@ -83,7 +83,7 @@ int adjoint_fused(wf_handle *h, const wf_adjoint_args *a, const wf::MetricDev<S>
   const size_t lds = lut ? table : 0;
   const int threads = 64 * (TY + 3);
   const int64_t conc = (int64_t)fused_occupancy(h, (const void *)kern, threads, lds) * h->ncu;
-  t.KZ = auto_kz((int64_t)t.ntx * t.nty, g.Nz, conc);
+  t.KZ = auto_kz((int64_t)t.ntx * t.nty, g.Nz, conc, h->ncu, threads / 64, (int)sizeof(A));
   t.ntz = (g.Nz + t.KZ - 1) / t.KZ;
   const int64_t nbf = (int64_t)t.ntx * t.nty * t.ntz;
   if (nbf > 2147483647LL) return fail(WF_ERANGE, "wf_adjoint_step: grid too large");

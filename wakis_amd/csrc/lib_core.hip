@@ -2,6 +2,7 @@
 // Handles, the exact step path, captures, wake post-processing and reductions.
 #include "lib_internal.h"
 
+#include <cmath>
 #include <mutex>
 #include "monitor.h"
 #include "reduce.h"
@@ -205,21 +206,30 @@ int fused_occupancy(wf_handle *h, const void *kern, int threads, size_t lds) {
   return per_cu;
 }
 
-// z-planes per workgroup. About 512 workgroups (long z marches, measured best),
-// KZ in [8, 64]; then, since each workgroup's march is a serial chain whose
-// time hardly depends on how many others run, a last round of workgroups that
-// would fill at most a quarter of the machine is avoided by the smallest
-// longer KZ that needs one round less.
-int auto_kz(int64_t nxy, int Nz, int64_t conc) {
-  const auto clampkz = [](int64_t k) { return (int)(k < 8 ? 8 : (k > 64 ? 64 : k)); };
-  const int kz0 = clampkz((Nz * nxy + 511) / 512);
-  const auto rounds = [&](int kz) { return (nxy * ((Nz + kz - 1) / kz) + conc - 1) / conc; };
-  const int64_t nwg = nxy * ((Nz + kz0 - 1) / kz0);
-  const int64_t r0 = rounds(kz0);
-  if (r0 < 2 || nwg - (r0 - 1) * conc > conc / 4) return kz0;
-  for (int kz = kz0 + 1; kz <= 64; ++kz)
-    if (rounds(kz) < r0) return kz;
-  return kz0;
+// z-planes per workgroup, KZ <= 64: the least time of the busiest CU. A
+// workgroup marches KZ + 1 planes, each a chain of loads and two barriers: one
+// workgroup on a CU takes the chain's time per plane, r of them the longer of it
+// and r times the share of it that their waves need (0.05 a wave and 0.0065 per
+// byte of a lane's row, at most 0.95: from 0.4 for 4 waves of one double on).
+// Within 4% of the best of KZ = 1 .. 64 on 20 grids of one step per launch and 6
+// of the reverse step (9% on one). The former rule, at least 8 planes per
+// workgroup, took 15.9 us per step against 7.9 at 40x40x64 FP32, 17.4 / 13.1 at
+// 48x48x128 FP64, 213 / 152 at 160x160x160 FP64, and 17.3 ms against 10.9 for the
+// 720 FP32 reverse steps at 64x64x96; from 256x256x256 on both are within 3%.
+int auto_kz(int64_t nxy, int Nz, int64_t conc, int ncu, int waves, int lane_bytes) {
+  const double share = std::min(0.95, waves * (0.05 + 0.0065 * lane_bytes));
+  const double per_cu = std::max<double>(1.0, (double)(conc / ncu));
+  double best = 1e300;
+  int kz = 1;
+  for (int k = 1; k <= std::min(Nz, 64); ++k) {
+    // workgroups on the busiest CU: at once or in two rounds, or in turn with a
+    // ragged end
+    const double n = (double)(nxy * ((Nz + k - 1) / k)) / ncu;
+    const double r = std::ceil(n) <= std::max(per_cu, 2.0) ? std::ceil(n) : n + 0.6;
+    const double t = (k + 1) * std::max(1.0, share * r);
+    if (t <= best) { best = t; kz = k; }
+  }
+  return kz;
 }
 
 // Argument checks shared by wf_step and wf_batch_create.

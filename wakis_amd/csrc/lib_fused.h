@@ -113,7 +113,8 @@ int step_fused4(wf_handle *h, wf_step_args *a, const wf::MetricDev<S> &m, hipStr
       const int64_t kz = ((int64_t)(hz - lz) * x.ntx * x.nty + conc - 1) / conc;
       x.KZ = (int)std::min<int64_t>(64, std::max<int64_t>(2, kz));
     } else {
-      x.KZ = auto_kz((int64_t)x.ntx * x.nty, g.Nz, conc);
+      x.KZ = auto_kz((int64_t)x.ntx * x.nty, g.Nz, conc, h->ncu, threads / 64,
+                     V * (int)sizeof(S));
     }
   }
   x.ntz = (g.Nz + x.KZ - 1) / x.KZ;

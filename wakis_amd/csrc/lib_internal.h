@@ -97,8 +97,9 @@ WF_HIDDEN void monitor_store(const wf_handle *h, const wf_step_args *a, const S 
 // Workgroups of `kern` that one CU runs at once (cached per handle).
 WF_HIDDEN int fused_occupancy(wf_handle *h, const void *kern, int threads, size_t lds);
 
-// z-planes per workgroup for nxy tiles per plane and `conc` resident workgroups.
-WF_HIDDEN int auto_kz(int64_t nxy, int Nz, int64_t conc);
+// z-planes per workgroup for nxy tiles per plane, `conc` resident workgroups of
+// `waves` waves on ncu CUs, a lane holding lane_bytes of a row.
+WF_HIDDEN int auto_kz(int64_t nxy, int Nz, int64_t conc, int ncu, int waves, int lane_bytes);
 
 // Full-row tiles: dynamic LDS bytes of a tile of `rows` own rows (E and H rows
 // of Nx + 2V slots, then the material table).
