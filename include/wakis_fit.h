@@ -175,18 +175,24 @@ typedef struct wf_step_args {
    * material codes with zero_masked and no escape code, the beam line fed
    * from beam_table (with or without conduction), row segments (variant 0,
    * full_rows <= 0, cells_per_lane 0 or 16 bytes of cells), every 3N array
-   * within 4 GiB, no box, no trajectory, no monitor; otherwise one step per
+   * within 4 GiB, no box, no trajectory, no monitor without mon_work; otherwise one step per
    * launch. Results are identical to one step per launch. 0 = one step per
    * launch; 4 or 8: two steps per launch with at most that many rows per
    * workgroup.
    * E2 and H2 hold the fields one step back after a call, except (fields two
    * steps back) after an even count with Nx <= 256 a multiple of 4 (FP64: 2)
    * and two_step 4 or 8, or 1 on grids of 2^20 cells or more (FP64 also
-   * Nx >= 224): such a call takes all its steps in pairs, every other one its
+   * Nx >= 224) and no monitor: such a call takes all its steps in pairs, every other its
    * last step or two singly. */
   int32_t two_step;
   int32_t two_step_used;  /* out: two steps per launch, 1: to the call's end (but an
                            * odd step), 2: up to its single last steps            */
+  /* Optional with mon_acc: device scratch of mon_slots (1, 3 or 7) times 3N
+   * values of the storage type. Where the two-step kernel applies, the
+   * accumulators then cross memory once per 2, 4 or 8 steps; same results, the
+   * call's last step or two singly. */
+  void *mon_work;
+  int32_t mon_slots;
 } wf_step_args;
 
 int wf_version(void);

@@ -283,6 +283,7 @@ int check_step_args(const wf_handle *h, const wf_step_args *a, const char *who) 
                      (a->mon_phase_f32 != 0 && a->mon_phase_f32 != 1)))
     return fail(WF_EINVAL, "%s: the field monitor needs a phase table, mon_nf >= 1, "
                 "mon_row0 >= 0 and mon_phase_f32 0 or 1", who);
+  if (a->mon_slots < 0) return fail(WF_EINVAL, "%s: mon_slots < 0", who);
   if (a->path == 1) {
     if (!a->E2 || !a->H2 || a->E2 == a->E || a->H2 == a->H || a->E2 == a->H2)
       return fail(WF_EINVAL, "%s: fused path needs distinct E2/H2 buffers", who);

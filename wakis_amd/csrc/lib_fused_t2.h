@@ -26,6 +26,23 @@ T2Fn<S> pick_t2(bool cond, bool desc, bool rag) {
 #undef WF_T2
 }
 
+template <typename S>
+using T2MonFn = void (*)(wf::GridDev, wf::MetricDev<S>, const S *, const S *, S *, S *, S *,
+                         wf::Coefs<S>, S, wf::T2Aux, const S *, const S *, S *, S *);
+
+template <typename S>
+T2MonFn<S> pick_t2_mon(bool cond, bool desc, bool rag) {
+#define WF_T2(CO, DE)                                                          \
+  return rag ? &wf::k_fused4_t2_mon<S, CO, DE, true> : &wf::k_fused4_t2_mon<S, CO, DE, false>
+  if (cond) {
+    if (desc) WF_T2(true, true);
+    WF_T2(true, false);
+  }
+  if (desc) WF_T2(false, true);
+  WF_T2(false, false);
+#undef WF_T2
+}
+
 // A tile shape of the two-step kernel and the z chunk of a launch.
 struct T2Shape {
   bool ok = false;
@@ -153,6 +170,34 @@ int launch_t2(wf_handle *h, wf_step_args *a, const wf::MetricDev<S> &m, hipStrea
   // or two when the spare buffers have to hold the fields one step back)
   const int paired = end_paired ? a->nsteps / 2 * 2 : (a->nsteps - 1) / 2 * 2;
   int cur = 0, s = 0;
+  // with a field monitor, the E of up to mon_slots + 1 steps in turn (a first
+  // step's and all but the last second step's in the work array), then one pass
+  // over the accumulators
+  if (a->mon_acc) {
+    const T2MonFn<S> mkern = pick_t2_mon<S>(cond, desc, rag);
+    const int per = std::min(wf::MON_STEPS, a->mon_slots + 1) / 2;  // pairs per pass
+    const auto slot = [&](int i) { return (S *)a->mon_work + (int64_t)i * 3 * g.N; };
+    while (s < paired) {
+      const int np = std::min(per, (paired - s) / 2);
+      wf::MonFields<S> f{};
+      const S *e = Ebuf[cur];
+      for (int p = 0; p < np; ++p, s += 2) {
+        S *e1 = slot(2 * p), *e2 = p + 1 < np ? slot(2 * p + 1) : Ebuf[(cur + np) & 1];
+        const S *row1 = table + (a->beam_row0 + s) * g.Nz;
+        x.cap_sample = a->cap_sample0 + s;
+        x.skip_j = 1;  // J = sigma E is stored by the single steps at the end
+        hipLaunchKernelGGL(mkern, dim3((unsigned)nb), dim3(threads), sh.lds, st, g, m, e,
+                           Hbuf[(cur + p) & 1], e2, Hbuf[(cur + p + 1) & 1], (S *)a->J, cf, dt, x,
+                           row1, row1 + g.Nz, (S *)a->capture, e1);
+        WF_LAUNCH_CHECK();
+        f.e[2 * p] = e1;
+        f.e[2 * p + 1] = e = e2;
+      }
+      monitor_steps<S>(h, a, f, s - 2 * np, 2 * np, st);
+      WF_LAUNCH_CHECK();
+      cur = (cur + np) & 1;
+    }
+  }
   for (; s < paired; s += 2) {
     const S *row1 = table ? table + (a->beam_row0 + s) * g.Nz : nullptr;
     const S *row2 = table ? table + (a->beam_row0 + s + 1) * g.Nz : nullptr;
@@ -170,6 +215,7 @@ int launch_t2(wf_handle *h, wf_step_args *a, const wf::MetricDev<S> &m, hipStrea
     b.nsteps = a->nsteps - s;
     b.beam_row0 = a->beam_row0 + s;
     b.cap_sample0 = a->cap_sample0 + s;
+    b.mon_row0 = a->mon_row0 + s;
     if (cur) {
       b.E = a->E2; b.E2 = a->E;
       b.H = a->H2; b.H2 = a->H;

@@ -19,18 +19,18 @@ int fused_t2_applies(const wf_handle *h, const wf_step_args *a) {
   if (a->two_step == 0 || !lut || !a->zero_masked || a->code_escape || a->compute_f64 || !jok ||
       (uint64_t)3 * (uint64_t)g.N * (uint64_t)elem >= (1ull << 32) || a->variant != 0 ||
       a->full_rows > 0 || (a->cells_per_lane != 0 && a->cells_per_lane != vn) || box ||
-      a->traj_E || a->mon_acc || a->nsteps < 2)
+      a->traj_E || (a->mon_acc && (!a->mon_work || a->mon_slots < 1)) || a->nsteps < 2)
     return 0;
   // Pairs are the faster launches at every size measured (us per step, one step
   // per launch against pairs: 32x32x64 FP32 16.0 / 7.5, 48x48x128 FP64 17.2 /
   // 9.5, 91x75x161 FP32 35.0 / 17.6, 160x160x200 FP64 267 / 77, 300x220x180
   // FP32 270 / 99). Where a call always ended with a single step, so that
   // the spare buffers hold the fields one step back, it still does: rows that
-  // are no whole number of lanes or longer than 256 cells and, by default (1),
-  // grids under 2^20 cells and FP64 rows under 224 cells.
+  // are no whole number of lanes or longer than 256 cells, runs with a field
+  // monitor and, by default (1), grids under 2^20 cells and FP64 rows under 224 cells.
   const bool big = a->two_step != 1 ||
                    (g.N >= (int64_t)1 << 20 && (h->dtype == WF_F32 || g.Nx >= 224));
-  if (big && g.Nx <= 256 && g.Nx % vn == 0) return 1;
+  if (big && g.Nx <= 256 && g.Nx % vn == 0 && !a->mon_acc) return 1;
   return a->nsteps >= 3 ? 2 : 0;
 }
 

@@ -94,6 +94,20 @@ WF_HIDDEN void monitor_store(const wf_handle *h, const wf_step_args *a, const S 
                  st);
 }
 
+// The same for the E of steps s .. s + nk - 1 of the call, in one pass.
+template <typename S>
+inline void monitor_steps(const wf_handle *h, const wf_step_args *a, const wf::MonFields<S> &f,
+                          int64_t s, int nk, hipStream_t st) {
+  const dim3 grid(nblocks(h->g.N, 256), 3);
+  const int64_t row = (a->mon_row0 + s) * 2 * a->mon_nf;
+  if (a->mon_phase_f32)
+    hipLaunchKernelGGL((wf::k_monitor_steps<S, float>), grid, dim3(256), 0, st, f, nk, h->g.N,
+                       (const float *)a->mon_phase + row, a->mon_nf, a->mon_acc);
+  else
+    hipLaunchKernelGGL((wf::k_monitor_steps<S, double>), grid, dim3(256), 0, st, f, nk, h->g.N,
+                       (const double *)a->mon_phase + row, a->mon_nf, a->mon_acc);
+}
+
 // Workgroups of `kern` that one CU runs at once (cached per handle).
 WF_HIDDEN int fused_occupancy(wf_handle *h, const void *kern, int threads, size_t lds);
 

@@ -33,4 +33,42 @@ k_monitor(const S *__restrict__ E, int64_t N, const P *__restrict__ phase, int n
   }
 }
 
+// The same for the E of nk <= MON_STEPS steps in turn: each accumulator crosses
+// memory once for all of them (16 bytes read and written per component,
+// frequency and cell, against 4 or 8 for a step's E), the sum in the same order.
+// Bound by those bytes: 96x96x160 FP32, 2 frequencies, 57 us for 8 steps at 7.4 TB/s
+// (the accumulators stay in the last cache), 46 us for one step before.
+constexpr int MON_STEPS = 8;
+template <typename S>
+struct MonFields {
+  const S *e[MON_STEPS];
+};
+
+template <typename S, typename P>
+__global__ void __launch_bounds__(256)
+k_monitor_steps(MonFields<S> E, int nk, int64_t N, const P *__restrict__ phase, int nf,
+                double *__restrict__ acc) {
+  using R = typename std::conditional<sizeof(S) == 4 && sizeof(P) == 4, float, double>::type;
+  const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (n >= N) return;
+  const int c = blockIdx.y;
+  R e[MON_STEPS];
+#pragma unroll
+  for (int k = 0; k < MON_STEPS; ++k) e[k] = k < nk ? (R)E.e[k][c * N + n] : R(0);
+  for (int f = 0; f < nf; ++f) {
+    double2 *a = reinterpret_cast<double2 *>(acc) + (((int64_t)c * nf + f) * N + n);
+    double2 s = *a;
+#pragma unroll
+    for (int k = 0; k < MON_STEPS; ++k) {
+      if (k >= nk) break;
+      const R re = (R)phase[2 * ((int64_t)k * nf + f)], im = (R)phase[2 * ((int64_t)k * nf + f) + 1];
+      const R pr = e[k] * re - R(0) * im;
+      const R pi = e[k] * im + R(0) * re;
+      s.x = s.x + (double)pr;
+      s.y = s.y + (double)pi;
+    }
+    *a = s;
+  }
+}
+
 }  // namespace wf

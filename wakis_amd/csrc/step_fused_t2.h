@@ -160,13 +160,13 @@ __host__ __device__ inline int t2_dyn_values(int V, int Q, int T, int KZ, int nm
   return 8 * Q * V + 6 * (T + 4) + 4 * (KZ + 3) + 9 * nmat;
 }
 
-template <typename S, bool COND, bool DESC, bool RAG>
+template <typename S, bool COND, bool DESC, bool RAG, bool MON = false>
 __device__ __forceinline__ void
 t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
         const S *__restrict__ Hin, S *__restrict__ Eout, S *__restrict__ Hout,
         S *__restrict__ J, const Coefs<S> &cf, S dt, const T2Aux &x,
         const S *__restrict__ beam1, const S *__restrict__ beam2, S *__restrict__ cap,
-        const int tile) {
+        const int tile, S *__restrict__ E1out = nullptr) {
   using I = uint32_t;  // byte offsets: every 3N array within 4 GiB
   constexpr int V = 16 / sizeof(S);
   constexpr int NM = 9;
@@ -458,6 +458,8 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
       }
       if (capq0 < capq1 && x.cap_sample < x.cap_samples && k >= k0 && k < kend)
         capture(k, E1[2]);
+      if (MON && k >= k0 && k < kend)  // E of the first step, for a field monitor
+        buf_st<RAG>(buf_of(E1out, 3 * NB), ofs, (I)k * sz * ES, NB, E1);
     }
     if (doH2 && p >= kstart) {  // H2 below plane 0 stays 0
       const S iaxp = rowv(0, rp), Lzp = plv(0, p);
@@ -581,6 +583,17 @@ k_fused4_t2(GridDev g, MetricDev<S> m, const S *__restrict__ Ein, const S *__res
             S *__restrict__ cap) {
   t2_tile<S, COND, DESC, RAG>(g, m, Ein, Hin, Eout, Hout, J, cf, dt, x, beam1, beam2, cap,
                              xcd_tile(blockIdx.x, x.ntx * x.nty * x.ntz));
+}
+
+// The same, the E of the first step stored too (E1out).
+template <typename S, bool COND, bool DESC, bool RAG>
+__global__ void __launch_bounds__(T2_NT)
+k_fused4_t2_mon(GridDev g, MetricDev<S> m, const S *__restrict__ Ein, const S *__restrict__ Hin,
+                S *__restrict__ Eout, S *__restrict__ Hout, S *__restrict__ J, Coefs<S> cf, S dt,
+                T2Aux x, const S *__restrict__ beam1, const S *__restrict__ beam2,
+                S *__restrict__ cap, S *__restrict__ E1out) {
+  t2_tile<S, COND, DESC, RAG, true>(g, m, Ein, Hin, Eout, Hout, J, cf, dt, x, beam1, beam2, cap,
+                                    xcd_tile(blockIdx.x, x.ntx * x.nty * x.ntz), E1out);
 }
 
 // One grid of a batch that takes its steps in pairs (BatchDesc) and its tiles.

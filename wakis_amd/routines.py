@@ -122,10 +122,9 @@ class RoutinesMixin:
             # long run: measure the kernel shapes first, unless it takes two steps
             # per launch, which no shape of one step per launch beats (the trials
             # took 44 of 712 ms of a 3,600-step run at 256x256x512)
-            mon = use_field_monitor and field_monitor is not None
             per_call = min(1 if callback is not None else Nt if chunk is None else int(chunk),
                            Nt if every is None else every)
-            if mon or per_call < 3 or not self._pairs_apply(self._wake_args(ctx, 0, 3)):
+            if per_call < 3 or not self._pairs_apply(self._wake_args(ctx, 0, 3)):
                 self.tune_fused(lambda k: self._wake_args(ctx, 0, k))
         if save_J:  # J_z on the window before the run, for Jz.h5
             ix0, iy0, nx, ny = ctx["win"]
@@ -135,6 +134,7 @@ class RoutinesMixin:
         print("Running electromagnetic time-domain simulation...")
         t0 = time.time()
         monitor = field_monitor if (use_field_monitor and field_monitor is not None) else None
+        work = self._monitor_work() if monitor is not None else None
         per_step = callback is not None
         step = 1 if per_step else (Nt if chunk is None else int(chunk))
         while n < Nt:
@@ -144,6 +144,8 @@ class RoutinesMixin:
             args = self._wake_args(ctx, n, k)
             if monitor is not None:  # accumulated after every step of the call
                 phases = monitor._step_args(args, self.E, self.dt, k)
+                if work is not None:
+                    args.mon_work, args.mon_slots = _lib.ptr(work), work.shape[0]
             self._run(args)
             self.nstep += k
             if monitor is not None:
@@ -155,6 +157,7 @@ class RoutinesMixin:
             if every is not None and n % every == 0 and n < Nt:
                 self._wake_checkpoint(ctx, checkpoint, n)
         torch.cuda.synchronize(self.device)
+        del work
         self.simulationTime = time.time() - t0
         self.fields_finite = self.check_finite(("E", "H"))
         if not self.fields_finite:

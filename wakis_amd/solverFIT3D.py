@@ -793,7 +793,19 @@ class SolverFIT3D(RoutinesMixin):
         return bool(args.two_step and args.code and args.zero_masked and not args.code_escape
                     and args.beam_table and 3 * self.N * size < 2 ** 32 and args.variant == 0
                     and args.full_rows <= 0 and args.cells_per_lane in (0, 16 // size)
-                    and not box and not args.traj_E and not args.mon_acc)
+                    and not box and not args.traj_E and (not args.mon_acc or args.mon_work))
+
+    def _monitor_work(self):
+        """Scratch for the E of up to eight steps of a monitored run (7, 3 or 1
+        arrays of 3N values, at most a quarter of the free device memory), or
+        None."""
+        free, _ = torch.cuda.mem_get_info(self.device)
+        one = self.E.array.numel() * self.E.array.element_size()
+        for slots in (7, 3, 1):
+            if slots * one <= free // 4:
+                return torch.empty((slots, self.E.array.numel()), dtype=self.E.array.dtype,
+                                   device=self.device)
+        return None
 
     def tune_fused(self, make_args=None, steps=3):
         """Choose the fused kernel's workgroup shape by timing it (no reference
