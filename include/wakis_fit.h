@@ -193,7 +193,18 @@ typedef struct wf_step_args {
    * call's last step or two singly. */
   void *mon_work;
   int32_t mon_slots;
+  /* Optional with code, FP32 storage, two steps per launch: per cell a weight
+   * code, a row of wtab (wf_weight_rows, wf_weight_codes; row 0 all zeros). The
+   * rows hold the products that the kernel otherwise forms at every cell; same
+   * results. */
+  const void *wcode;      /* device uint8[N]                                          */
+  const void *wtab;       /* device FP32 [nw][WF_WEIGHT_ROW]                          */
+  int32_t nw;             /* 1..256                                                   */
 } wf_step_args;
+
+/* Values of a row of the weight table: the 6 weights of the H rows, the 6 of
+ * the E rows, ieps and sigma per component, 2 unused. */
+#define WF_WEIGHT_ROW 20
 
 int wf_version(void);
 const char *wf_last_error(void);
@@ -201,6 +212,21 @@ const char *wf_last_error(void);
 /* Replaces SolverFIT3D.__init__'s operator set-up (solverFIT3D.py:203-227). */
 int wf_create(const wf_grid *g, wf_handle **out);
 int wf_destroy(wf_handle *h);
+
+/* Weights of the cells of a grid on FP32 material codes whose metric is the
+ * same for all cells of a class: the first, the inner and the last cells of an
+ * axis (uniform spacing). For class c = cx + 3 (cy + 3 cz) and material code m,
+ * rows[(c * nmat + m)][WF_WEIGHT_ROW] gets the weights dt fl(a L) of the H rows,
+ * b tL of the E rows, ieps and sigma, and used[c * nmat + m] is 1 if any cell
+ * has them; used[27 * nmat] is nonzero if the metric differs within a class
+ * (no weights then). metric2d as in wf_step_args, with zero_masked. Device
+ * buffers: rows FP32 [27 * nmat][WF_WEIGHT_ROW], used int32 [27 * nmat + 1]. */
+int wf_weight_rows(wf_handle *h, const void *code, const void *mat, int32_t nmat,
+                   const void *metric2d, double dt, void *rows, int32_t *used, void *stream);
+
+/* wcode[n] = map[c * nmat + code[n]] of every cell (device uint8 buffers). */
+int wf_weight_codes(wf_handle *h, const void *code, int32_t nmat, const uint8_t *map,
+                    uint8_t *wcode, void *stream);
 
 /* First-step ghost zeroing, SolverFIT3D._set_ghosts_to_0 (solverFIT3D.py:820-840). */
 int wf_zero_ghosts(wf_handle *h, void *E, void *H, void *stream);

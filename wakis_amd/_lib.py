@@ -13,6 +13,7 @@ LIB_PATH = Path(__file__).resolve().with_name("libwakis_fit.so")
 WF_OK, WF_EINVAL, WF_ERANGE, WF_EHIP, WF_ESTATE = 0, -1, -2, -3, -4
 WF_F64, WF_F32 = 0, 1
 WF_J_NONE, WF_J_LINE, WF_J_FULL = 0, 1, 2
+WF_WEIGHT_ROW = 20
 
 
 class WfGrid(ctypes.Structure):
@@ -46,6 +47,7 @@ class WfStepArgs(ctypes.Structure):
         ("mon_acc", c_void_p), ("mon_phase", c_void_p), ("mon_row0", c_int64),
         ("mon_nf", c_int32), ("mon_phase_f32", c_int32), ("two_step", c_int32),
         ("two_step_used", c_int32), ("mon_work", c_void_p), ("mon_slots", c_int32),
+        ("wcode", c_void_p), ("wtab", c_void_p), ("nw", c_int32),
     ]
 
 
@@ -84,6 +86,9 @@ EXPORTS = {
     "wf_last_error": (ctypes.c_char_p, []),
     "wf_create": (c_int32, [POINTER(WfGrid), POINTER(c_void_p)]),
     "wf_destroy": (c_int32, [c_void_p]),
+    "wf_weight_rows": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_void_p, c_double,
+                                 c_void_p, c_void_p, c_void_p]),
+    "wf_weight_codes": (c_int32, [c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_void_p]),
     "wf_zero_ghosts": (c_int32, [c_void_p, c_void_p, c_void_p, c_void_p]),
     "wf_step": (c_int32, [c_void_p, POINTER(WfStepArgs), c_void_p]),
     "wf_capture": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32,

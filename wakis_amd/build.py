@@ -24,7 +24,7 @@ SOURCES = ["lib_fused_f32_a.hip", "lib_fused_f32_b.hip", "lib_fused_f32_c.hip",
 HEADERS = ["lib_internal.h", "lib_fused.h", "lib_fused_t2.h", "fit_common.h",
            "step_general.h", "step_fused.h",
            "step_fused4.h", "step_fused_t2.h", "wake.h", "reduce.h", "adjoint.h",
-           "adjoint_fused.h", "monitor.h"]
+           "adjoint_fused.h", "monitor.h", "weight_codes.h"]
 
 # -ffp-contract=off keeps every multiply and add separately rounded, as numpy
 # and scipy's csr_matvec do on the host; -packed-fp32-ops keeps the compiler

@@ -12,14 +12,24 @@ int build(const wf::BatchDesc<S> *bd, wf_handle *const *hs, const wf_step_args *
   double cells = 0;
   for (int i = 0; i < n; ++i) cells += (double)hs[i]->g.N;
   int64_t tiles = 0;
+  t->wc = 1;
+  for (int i = 0; i < n; ++i)
+    if (!wff::t2_weights(hs[i], &as[i])) t->wc = 0;
   for (int i = 0; i < n; ++i) {
     const wf::GridDev &g = hs[i]->g;
     // the grid's share of the CUs
     const int share = std::max(1, (int)std::lround(BATCH_T2_LOAD * ncu * (double)g.N / cells));
-    const wff::T2Shape sh = wff::t2_shape<S>(g, as[i].nmat, std::min(share, ncu), 0, 0,
+    const wff::T2Shape sh = wff::t2_shape<S>(g, t->wc ? as[i].nw : as[i].nmat, t->wc != 0,
+                                             std::min(share, ncu), 0, 0,
                                              std::max(0, ncu - share));
     if (!sh.ok) return 0;
     d[i].b = bd[i];
+    if (t->wc) {
+      wf::Coefs<S> &cf = d[i].b.cf;
+      cf.code = (const uint8_t *)as[i].wcode;
+      cf.mat = (const S *)as[i].wtab;
+      cf.nmat = as[i].nw;
+    }
     wff::t2_aux(sh, g, &as[i], d[i].x);
     d[i].tile0 = (int)tiles;
     tiles += (int64_t)d[i].x.ntx * d[i].x.nty * d[i].x.ntz;
@@ -37,14 +47,21 @@ int build(const wf::BatchDesc<S> *bd, wf_handle *const *hs, const wf_step_args *
 template <typename S>
 void launch(const batch_t2 *t, int n, int cond, int desc, int s, int step0, int end, int flip,
             hipStream_t st) {
-#define WF_BT2(CO, DE, RA)                                                                       \
-  hipLaunchKernelGGL((wf::k_fused4_t2_batch<S, CO, DE, RA>), dim3((unsigned)t->ntiles),          \
+#define WF_BT2(CO, DE, RA, WC)                                                                   \
+  hipLaunchKernelGGL((wf::k_fused4_t2_batch<S, CO, DE, RA, WC>), dim3((unsigned)t->ntiles),      \
                      dim3(t->threads), t->lds, st, (const wf::T2Batch<S> *)t->desc_dev, n,       \
                      t->ntiles, s, step0, end, flip)
 #define WF_BT2R(CO, DE)                                                                          \
   do {                                                                                           \
-    if (t->rag) WF_BT2(CO, DE, true);                                                            \
-    else WF_BT2(CO, DE, false);                                                                  \
+    if constexpr (sizeof(S) == 4) {                                                              \
+      if (t->wc) {                                                                               \
+        if (t->rag) WF_BT2(CO, DE, true, true);                                                  \
+        else WF_BT2(CO, DE, false, true);                                                        \
+        break;                                                                                   \
+      }                                                                                          \
+    }                                                                                            \
+    if (t->rag) WF_BT2(CO, DE, true, false);                                                     \
+    else WF_BT2(CO, DE, false, false);                                                           \
   } while (0)
   if (cond) {
     if (desc) WF_BT2R(true, true);

@@ -7,6 +7,7 @@
 #include "monitor.h"
 #include "reduce.h"
 #include "wake.h"
+#include "weight_codes.h"
 
 namespace {
 thread_local std::string g_err;
@@ -129,6 +130,38 @@ int wf_destroy(wf_handle *h) {
   if (h->metric_buf) hipFree(h->metric_buf);
   if (h->red_buf) hipFree(h->red_buf);
   delete h;
+  return WF_OK;
+}
+
+int wf_weight_rows(wf_handle *h, const void *code, const void *mat, int32_t nmat,
+                   const void *metric2d, double dt, void *rows, int32_t *used, void *stream) {
+  if (!h || !code || !mat || !metric2d || !rows || !used)
+    return fail(WF_EINVAL, "wf_weight_rows: null argument");
+  if (h->dtype != WF_F32) return fail(WF_EINVAL, "wf_weight_rows: FP32 storage only");
+  if (nmat < 1 || nmat > 256) return fail(WF_EINVAL, "wf_weight_rows: nmat must be 1..256");
+  hipStream_t st = (hipStream_t)stream;
+  const int nkeys = 27 * nmat;
+  hipLaunchKernelGGL(wf::k_weight_rows<float>, dim3(nblocks(nkeys, 256)), dim3(256), 0, st, h->g,
+                     h->mf, (const float *)mat, nmat, (const float *)metric2d, (float)dt,
+                     (float *)rows, used);
+  WF_LAUNCH_CHECK();
+  const int64_t wgs = std::min<int64_t>((int64_t)h->ncu * 4, nblocks(h->g.N, 256));
+  hipLaunchKernelGGL(wf::k_weight_scan<float>, dim3((unsigned)wgs), dim3(256),
+                     sizeof(int) * (nkeys + 1), st, h->g, h->mf, (const uint8_t *)code, nmat,
+                     (const float *)metric2d, used);
+  WF_LAUNCH_CHECK();
+  return WF_OK;
+}
+
+int wf_weight_codes(wf_handle *h, const void *code, int32_t nmat, const uint8_t *map,
+                    uint8_t *wcode, void *stream) {
+  if (!h || !code || !map || !wcode) return fail(WF_EINVAL, "wf_weight_codes: null argument");
+  if (nmat < 1 || nmat > 256) return fail(WF_EINVAL, "wf_weight_codes: nmat must be 1..256");
+  const int64_t rows = (int64_t)h->g.Ny * h->g.Nz;
+  hipLaunchKernelGGL(wf::k_weight_codes, dim3((unsigned)std::min<int64_t>(nblocks(rows, 4), 65536)),
+                     dim3(256), 0, (hipStream_t)stream, h->g, (const uint8_t *)code, nmat, map,
+                     wcode);
+  WF_LAUNCH_CHECK();
   return WF_OK;
 }
 
@@ -283,6 +316,8 @@ int check_step_args(const wf_handle *h, const wf_step_args *a, const char *who) 
                      (a->mon_phase_f32 != 0 && a->mon_phase_f32 != 1)))
     return fail(WF_EINVAL, "%s: the field monitor needs a phase table, mon_nf >= 1, "
                 "mon_row0 >= 0 and mon_phase_f32 0 or 1", who);
+  if (a->wcode && (!a->wtab || a->nw < 1 || a->nw > 256))
+    return fail(WF_EINVAL, "%s: weight codes need a table of 1..256 rows", who);
   if (a->mon_slots < 0) return fail(WF_EINVAL, "%s: mon_slots < 0", who);
   if (a->path == 1) {
     if (!a->E2 || !a->H2 || a->E2 == a->E || a->H2 == a->H || a->E2 == a->H2)

@@ -14,9 +14,16 @@ using T2Fn = void (*)(wf::GridDev, wf::MetricDev<S>, const S *, const S *, S *, 
                       wf::Coefs<S>, S, wf::T2Aux, const S *, const S *, S *);
 
 template <typename S>
-T2Fn<S> pick_t2(bool cond, bool desc, bool rag) {
+T2Fn<S> pick_t2(bool cond, bool desc, bool rag, bool wc) {
 #define WF_T2(CO, DE)                                                                          \
-  return rag ? &wf::k_fused4_t2<S, CO, DE, true> : &wf::k_fused4_t2<S, CO, DE, false>
+  do {                                                                                         \
+    if constexpr (sizeof(S) == 4)                                                              \
+      if (wc)                                                                                  \
+        return rag ? &wf::k_fused4_t2<S, CO, DE, true, true>                                   \
+                   : &wf::k_fused4_t2<S, CO, DE, false, true>;                                 \
+    return rag ? &wf::k_fused4_t2<S, CO, DE, true, false>                                      \
+               : &wf::k_fused4_t2<S, CO, DE, false, false>;                                    \
+  } while (0)
   if (cond) {
     if (desc) WF_T2(true, true);
     WF_T2(true, false);
@@ -31,9 +38,16 @@ using T2MonFn = void (*)(wf::GridDev, wf::MetricDev<S>, const S *, const S *, S 
                          wf::Coefs<S>, S, wf::T2Aux, const S *, const S *, S *, S *);
 
 template <typename S>
-T2MonFn<S> pick_t2_mon(bool cond, bool desc, bool rag) {
-#define WF_T2(CO, DE)                                                          \
-  return rag ? &wf::k_fused4_t2_mon<S, CO, DE, true> : &wf::k_fused4_t2_mon<S, CO, DE, false>
+T2MonFn<S> pick_t2_mon(bool cond, bool desc, bool rag, bool wc) {
+#define WF_T2(CO, DE)                                                                          \
+  do {                                                                                         \
+    if constexpr (sizeof(S) == 4)                                                              \
+      if (wc)                                                                                  \
+        return rag ? &wf::k_fused4_t2_mon<S, CO, DE, true, true>                               \
+                   : &wf::k_fused4_t2_mon<S, CO, DE, false, true>;                             \
+    return rag ? &wf::k_fused4_t2_mon<S, CO, DE, true, false>                                  \
+               : &wf::k_fused4_t2_mon<S, CO, DE, false, false>;                                \
+  } while (0)
   if (cond) {
     if (desc) WF_T2(true, true);
     WF_T2(true, false);
@@ -67,7 +81,7 @@ constexpr size_t t2_static_lds() {
 // it picks is within 2% of the best measured one on average, 9% at most.
 // `others`: workgroups of other grids on the machine beside these.
 template <typename S>
-T2Shape t2_shape(const wf::GridDev &g, int nmat, int ncu, int want_rows, int want_kz,
+T2Shape t2_shape(const wf::GridDev &g, int nmat, bool wc, int ncu, int want_rows, int want_kz,
                  int others = 0) {
   constexpr int V = 16 / (int)sizeof(S);
   using C = wf::T2Slots;
@@ -102,10 +116,10 @@ T2Shape t2_shape(const wf::GridDev &g, int nmat, int ncu, int want_rows, int wan
         s.KZ = want_kz ? std::min(want_kz, g.Nz) : (int)std::max<int64_t>(1, (g.Nz + ntz - 1) / ntz);
         // the planes whose scalars (four a plane) fit beside the rest
         const int64_t room = ((int64_t)T2_LDS_CU - (int64_t)t2_static_lds<S>()) / (int64_t)sizeof(S);
-        const int64_t kz_max = (room - wf::t2_dyn_values(V, Q, s.T, 0, nmat)) / 4;
+        const int64_t kz_max = (room - wf::t2_dyn_values(V, Q, s.T, 0, nmat, wc)) / 4;
         if (kz_max < 1) continue;
         s.KZ = (int)std::min<int64_t>(s.KZ, kz_max);
-        s.lds = (size_t)wf::t2_dyn_values(V, Q, s.T, s.KZ, nmat) * sizeof(S);
+        s.lds = (size_t)wf::t2_dyn_values(V, Q, s.T, s.KZ, nmat, wc) * sizeof(S);
         const int64_t wgs = tiles * ((g.Nz + s.KZ - 1) / s.KZ);
         const int64_t rounds = (wgs + ncu - 1) / ncu;
         // us of a plane: the instructions of the four updates (whole waves of
@@ -124,6 +138,11 @@ T2Shape t2_shape(const wf::GridDev &g, int nmat, int ncu, int want_rows, int wan
   return out;
 }
 
+// whether pairs of steps run on weight codes: FP32 with a table of them
+inline bool t2_weights(const wf_handle *h, const wf_step_args *a) {
+  return h->dtype == WF_F32 && a->wcode && a->wtab && a->nw > 0;
+}
+
 inline void t2_aux(const T2Shape &sh, const wf::GridDev &g, const wf_step_args *a, wf::T2Aux &x) {
   x.ixs = a->ixs;
   x.iys = a->iys;
@@ -140,7 +159,10 @@ int launch_t2(wf_handle *h, wf_step_args *a, const wf::MetricDev<S> &m, hipStrea
               bool end_paired) {
   const wf::GridDev &g = h->g;
   constexpr int V = 16 / (int)sizeof(S);
-  const T2Shape sh = t2_shape<S>(g, a->nmat, h->ncu, a->two_step > 1 ? a->two_step : 0, a->kz);
+  const bool wc = t2_weights(h, a);
+  const int nrows = wc ? a->nw : a->nmat;
+  const T2Shape sh =
+      t2_shape<S>(g, nrows, wc, h->ncu, a->two_step > 1 ? a->two_step : 0, a->kz);
   if (!sh.ok) {  // one step per launch
     a->two_step = 0;
     return sizeof(S) == 4 ? step_fused_f32(h, a, st) : step_fused_f64(h, a, st);
@@ -148,14 +170,15 @@ int launch_t2(wf_handle *h, wf_step_args *a, const wf::MetricDev<S> &m, hipStrea
   wf::T2Aux x{};
   t2_aux(sh, g, a, x);
   const bool rag = g.Nx % V != 0, cond = a->conductive != 0, desc = g.m1desc != 0;
-  const T2Fn<S> kern = pick_t2<S>(cond, desc, rag);
+  const T2Fn<S> kern = pick_t2<S>(cond, desc, rag, wc);
   const int threads = ((sh.T + 4) * sh.Q + 63) / 64 * 64;
   const int64_t nb = (int64_t)x.ntx * x.nty * x.ntz;
   if (nb > 2147483647LL) return fail(WF_ERANGE, "wf_step: grid too large for the fused path");
   wf::Coefs<S> cf;
   cf.a = (const S *)a->a; cf.b = (const S *)a->b;
   cf.ieps = (const S *)a->ieps; cf.sigma = (const S *)a->sigma;
-  cf.code = (const uint8_t *)a->code; cf.mat = (const S *)a->mat; cf.nmat = a->nmat;
+  cf.code = (const uint8_t *)(wc ? a->wcode : a->code);
+  cf.mat = (const S *)(wc ? a->wtab : a->mat); cf.nmat = nrows;
   {
     const S *t = (const S *)a->metric2d;
     const int64_t yz = (int64_t)g.Ny * g.Nz, xz = (int64_t)g.Nx * g.Nz, xy = (int64_t)g.Nx * g.Ny;
@@ -174,7 +197,7 @@ int launch_t2(wf_handle *h, wf_step_args *a, const wf::MetricDev<S> &m, hipStrea
   // step's and all but the last second step's in the work array), then one pass
   // over the accumulators
   if (a->mon_acc) {
-    const T2MonFn<S> mkern = pick_t2_mon<S>(cond, desc, rag);
+    const T2MonFn<S> mkern = pick_t2_mon<S>(cond, desc, rag, wc);
     const int per = std::min(wf::MON_STEPS, a->mon_slots + 1) / 2;  // pairs per pass
     const auto slot = [&](int i) { return (S *)a->mon_work + (int64_t)i * 3 * g.N; };
     while (s < paired) {

@@ -152,6 +152,7 @@ WF_HIDDEN int step_fused_f64(wf_handle *h, wf_step_args *a, hipStream_t st);
 struct batch_t2 {
   void *desc_dev = nullptr;  // T2Batch<S>[n]
   int ntiles = 0, threads = 0, rag = 0;
+  int wc = 0;  // every grid has weight codes
   size_t lds = 0;
 };
 // 1 built, 0 no tile fits a grid (one step per launch then), < 0 an error

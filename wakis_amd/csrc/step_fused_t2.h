@@ -41,18 +41,25 @@
 // lanes (no bank conflicts). E and H are read once and written once per two
 // steps.
 //
-// What bounds it: the instructions its 12 waves issue (664 of 1,110 a plane are
-// the arithmetic of the exact row sums, FP32), and on large FP32 grids the
-// memory beside it. One branch per update and none per cell, buffer loads that
-// return zeros off the grid, own neighbours from registers: 16% fewer
-// instructions than the first form of this kernel (rows of one wave, a branch
-// per cell). us per step, that form -> this one: 256x256x512 FP32 197 -> 188
-// (1.70 GB per launch at 4.5 TB/s), 200x200x400 FP32 with conduction 149 ->
-// 111, 256x256x128 FP64 134 -> 106; and against one step per launch, which
-// other rows took: 160x160x200 FP64 267 -> 77, 300x220x180 FP32 270 -> 99,
-// 91x75x161 FP32 35 -> 17.6, 48x48x128 FP64 17.2 -> 9.4.
+// On weight codes (FP32, weight_codes.h) a cell's code names a row of finished
+// weights in LDS: 6 values for its H rows and 6 for its E rows in two reads
+// each, no metric values, rings or scalars beside them; the row 0 of zeros stands
+// for cells off the grid.
+//
+// What bounds it: on material codes the instructions its 12 waves issue (664 of
+// 1,110 a plane are the arithmetic of the exact row sums, FP32); on weight codes
+// (408 of 663) the chain of loads, LDS passes and barriers of a plane beside the
+// memory. One branch per update and none per cell, buffer loads that return zeros
+// off the grid, own neighbours from registers. us per step, rows of one wave and
+// a branch per cell -> this form on material codes -> on weight codes:
+// 256x256x512 FP32 197 -> 188 -> 178 (1.70 GB per launch at 4.8 TB/s),
+// 200x200x400 FP32 with conduction 149 -> 111 -> 98, 256x256x128 FP64 134 ->
+// 106; and against one step per launch, which other rows took: 160x160x200 FP64
+// 267 -> 77, 300x220x180 FP32 270 -> 99 -> 90, 91x75x161 FP32 35 -> 17.6 -> 15.1,
+// 48x48x128 FP64 17.2 -> 9.4.
 #pragma once
 #include "step_fused4.h"
+#include "weight_codes.h"
 
 namespace wf {
 
@@ -155,12 +162,40 @@ __device__ __forceinline__ void buf_st(Buf b, const Offs<V> &o, uint32_t s, uint
 
 // Dynamic LDS of a workgroup in values of S: the ring of iAy / itAy rows, the
 // x metric, the ring of iAx / itAx values, the per-plane scalars, the material
-// table.
-__host__ __device__ inline int t2_dyn_values(int V, int Q, int T, int KZ, int nmat) {
+// table; on weight codes the table of weights and the beam.
+__host__ __device__ inline int t2_dyn_values(int V, int Q, int T, int KZ, int nmat, bool wc) {
+  if (wc) return WC_ROW * nmat + 2 * (KZ + 3);
   return 8 * Q * V + 6 * (T + 4) + 4 * (KZ + 3) + 9 * nmat;
 }
 
-template <typename S, bool COND, bool DESC, bool RAG, bool MON = false>
+// The rows of h_row and e_sum with their weights given (w0 of terms 0 and 1, w1
+// of terms 2 and 3) and without the first addition to zero, which changes no
+// value but the sign of a zero sum: an H or E that is not -0 itself stays the
+// same bit for bit.
+template <bool DESC, typename S>
+__device__ __forceinline__ S t2_h(S h, S w0, S w1, S e0, S e1, S e2, S e3, int s0, int s2) {
+  const S p0 = w0 * e0, p1 = w0 * e1, p2 = w1 * e2, p3 = w1 * e3;
+  S acc;
+  if (!DESC) {
+    acc = s0 > 0 ? p0 - p1 : p1 - p0;
+    acc = s2 > 0 ? acc + p2 : acc - p2;
+    acc = s2 > 0 ? acc - p3 : acc + p3;
+  } else {
+    acc = s2 > 0 ? p2 - p3 : p3 - p2;
+    acc = s0 > 0 ? acc - p1 : acc + p1;
+    acc = s0 > 0 ? acc + p0 : acc - p0;
+  }
+  return h - acc;
+}
+template <typename S>
+__device__ __forceinline__ S t2_e(S w0, S w1, S h0, S h1, S h2, S h3, int s0, int s2) {
+  const S p0 = w0 * h0, p1 = w0 * h1, p2 = w1 * h2, p3 = w1 * h3;
+  S acc = s0 > 0 ? p0 - p1 : p1 - p0;
+  acc = s2 > 0 ? acc + p2 : acc - p2;
+  return s2 > 0 ? acc - p3 : acc + p3;
+}
+
+template <typename S, bool COND, bool DESC, bool RAG, bool WC, bool MON = false>
 __device__ __forceinline__ void
 t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
         const S *__restrict__ Hin, S *__restrict__ Eout, S *__restrict__ Hout,
@@ -169,7 +204,8 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
         const int tile, S *__restrict__ E1out = nullptr) {
   using I = uint32_t;  // byte offsets: every 3N array within 4 GiB
   constexpr int V = 16 / sizeof(S);
-  constexpr int NM = 9;
+  // a row of the table: 9 material values, or (WC) 12 weights, ieps, sigma
+  constexpr int NM = WC ? WC_ROW : 9, IE = WC ? 12 : 3, SG = WC ? 15 : 6;
   constexpr int CE0 = T2Slots::E0, CH1 = T2Slots::H1, CE1 = T2Slots::E1, CH2 = T2Slots::H2;
   // blocks [component][cell of the lane][slot]; the slot of lane ln of row r is
   // r * QS + ln + 1; a slot that no lane owns stays 0. Of H_y only the last
@@ -180,11 +216,13 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
   __shared__ S sH2_[(2 * V + 1) * CH2];  // H2(k-1), rows j0-1 .. j0+T-1
   extern __shared__ __align__(16) unsigned char s_dyn[];
   const int Q = x.Q, QS = x.QS, T = x.T;
-  S *sCy = reinterpret_cast<S *>(s_dyn);  // [plane % 3][iAy, itAy][Q * V]
+  S *sDyn = reinterpret_cast<S *>(s_dyn);
+  S *sCy = sDyn;                          // [plane % 3][iAy, itAy][Q * V]
   S *sX = sCy + 3 * 2 * Q * V;            // [Lx, tLx][Q * V]
   S *sRow = sX + 2 * Q * V;               // [plane % 3][iAx, itAx][T + 4]
-  S *sPl = sRow + 3 * 2 * (T + 4);        // [Lz, tLz, beam 1, beam 2][KZ + 3]
-  S *sMat = sPl + 4 * (x.KZ + 3);         // [nmat][9]
+  // [Lz, tLz, beam 1, beam 2][KZ + 3], the beams alone on weight codes
+  S *sPl = WC ? sDyn + NM * cf.nmat : sRow + 3 * 2 * (T + 4);
+  S *sMat = WC ? sDyn : sPl + 4 * (x.KZ + 3);  // [nmat][NM]
   typedef S vec __attribute__((ext_vector_type(V)));
   const auto ldsv = [&](const S *p, S (&o)[V]) {
     const vec v = *reinterpret_cast<const vec *>(p);
@@ -264,15 +302,18 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
   const auto h1 = [&](int c, int s, int q) -> S & { return sH1_[hb(c, q) * CH1 + s]; };
   const auto h2 = [&](int c, int s, int q) -> S & { return sH2_[hb(c, q) * CH2 + s]; };
 
-  if (r < 2) {
+  if (!WC && r < 2) {
 #pragma unroll
     for (int q = 0; q < V; ++q)
       sX[(r * Q + ln) * V + q] = q < nvx ? (r == 0 ? m.Lx : m.tLx)[xi + q] : S(0);
   }
-  S iAz[1][V], itAz[1][V];
-  buf_ld<RAG>(bM, of, true, (yz + xz) * ES, 0, iAz);
-  buf_ld<RAG>(bM, of, true, (2 * (yz + xz) + xy) * ES, 0, itAz);
-  const S Ly = rowok ? m.Ly[j] : S(0), tLy = rowok ? m.tLy[j] : S(0);
+  S iAz[1][V] = {}, itAz[1][V] = {};
+  S Ly = S(0), tLy = S(0);
+  if constexpr (!WC) {
+    buf_ld<RAG>(bM, of, true, (yz + xz) * ES, 0, iAz);
+    buf_ld<RAG>(bM, of, true, (2 * (yz + xz) + xy) * ES, 0, itAz);
+    if (rowok) { Ly = m.Ly[j]; tLy = m.tLy[j]; }
+  }
   const int qbeam = (lact && j == x.iys && x.ixs >= xi && x.ixs < xi + nv) ? x.ixs - xi : -1;
   // Ez window capture: own cells only, one sample per level
   int capq0 = V, capq1 = 0;
@@ -295,8 +336,9 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
   // per-plane values of planes kstart .. kend, staged once: Lz, tLz, the beam
   // of both levels
   const int NP = x.KZ + 3;
-  for (int t = threadIdx.x; t < 4 * NP; t += blockDim.x) {
-    const int which = t / NP, kk = kstart + t - which * NP;
+  constexpr int PL0 = WC ? 2 : 0;  // the first of the four that is staged
+  for (int t = threadIdx.x; t < (4 - PL0) * NP; t += blockDim.x) {
+    const int which = PL0 + t / NP, kk = kstart + t % NP;
     S v = S(0);
     if (kk < g.Nz && kk <= kend) {
       if (which == 0) v = m.Lz[kk];
@@ -306,9 +348,8 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
     }
     sPl[t] = v;
   }
-  const auto plv = [&](int which, int kk) { return sPl[which * NP + kk - kstart]; };
+  const auto plv = [&](int which, int kk) { return sPl[(which - PL0) * NP + kk - kstart]; };
   const auto ring = [](int kk) { return (kk + 3) % 3; };
-  const auto rowv = [&](int which, int slot) { return sRow[(slot * 2 + which) * (T + 4) + r]; };
   const auto cyv = [&](int which, int slot) { return sCy + ((slot * 2 + which) * Q + ln) * V; };
   // planes past the grid are zeros
   const auto load_e = [&](int kk, S (&o)[3][V]) {
@@ -332,11 +373,60 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
     }
     return c;
   };
+  // the weights of cell q's H rows (x: Ly, Lz; y: Lx, Lz; z: Lx, Ly) and E rows
+  // (the same of tL) at a lane's codes: from the table, or formed from the
+  // material values and the metric rows of the plane at ring slot rs
+  struct Metric {
+    S ax, z, cy[V], x[V];
+  };
+  const auto trow = [&](uint32_t cd, int q) {
+    return sMat + NM * (int)((cd >> (8 * q)) & 0xffu);
+  };
+  // which: 0 for H (iA, L), 1 for E (itA, tL)
+  const auto metric = [&](int which, int rs, int kk) {
+    Metric o = {};
+    if constexpr (!WC) {
+      o.ax = sRow[(rs * 2 + which) * (T + 4) + r];
+      o.z = sPl[which * NP + kk - kstart];
+      ldsv(sCy + ((rs * 2 + which) * Q + ln) * V, o.cy);
+      ldsv(sX + (which * Q + ln) * V, o.x);
+    }
+    return o;
+  };
+  const auto h_w = [&](const S *t, int q, const Metric &o, S (&w)[6]) {
+    if constexpr (WC) {
+      typedef S v4 __attribute__((ext_vector_type(4)));
+      typedef S v2 __attribute__((ext_vector_type(2)));
+      const v4 u = *reinterpret_cast<const v4 *>(t);
+      const v2 y = *reinterpret_cast<const v2 *>(t + 4);
+      w[0] = u[0]; w[1] = u[1]; w[2] = u[2]; w[3] = u[3]; w[4] = y[0]; w[5] = y[1];
+    } else {
+      const S a0 = (S)(o.ax * t[0]), a1 = (S)(o.cy[q] * t[1]), a2 = (S)(iAz[0][q] * t[2]);
+      w[0] = dt * (S)(a0 * Ly); w[1] = dt * (S)(a0 * o.z);
+      w[2] = dt * (S)(a1 * o.x[q]); w[3] = dt * (S)(a1 * o.z);
+      w[4] = dt * (S)(a2 * o.x[q]); w[5] = dt * (S)(a2 * Ly);
+    }
+  };
+  const auto e_w = [&](const S *t, int q, const Metric &o, S (&w)[6]) {
+    if constexpr (WC) {
+      typedef S v4 __attribute__((ext_vector_type(4)));
+      typedef S v2 __attribute__((ext_vector_type(2)));
+      const v2 y = *reinterpret_cast<const v2 *>(t + 6);
+      const v4 u = *reinterpret_cast<const v4 *>(t + 8);
+      w[0] = y[0]; w[1] = y[1]; w[2] = u[0]; w[3] = u[1]; w[4] = u[2]; w[5] = u[3];
+    } else {
+      const S b0 = (S)(t[3] * o.ax), b1 = (S)(t[4] * o.cy[q]), b2 = (S)(t[5] * itAz[0][q]);
+      w[0] = b0 * tLy; w[1] = b0 * o.z;
+      w[2] = b1 * o.x[q]; w[3] = b1 * o.z;
+      w[4] = b2 * o.x[q]; w[5] = b2 * tLy;
+    }
+  };
   struct Row {
     S cy[1][V], ax, bx;
   };
   // the metric rows of plane kk, and their place in the rings
   const auto load_row = [&](int kk, Row &o) {
+    if constexpr (WC) return;
     const bool in = kk < g.Nz;
     buf_ld<RAG>(bM, ofy, in, (I)kk * (I)g.Nx * ES, 0, o.cy);
     const I v = in ? vx : OOB, s = in ? (I)kk * (I)g.Ny * ES : 0;
@@ -344,6 +434,7 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
     o.bx = buf_ld1<S>(bM, v, s + (yz + xz + xy) * ES);
   };
   const auto put_row = [&](int kk, const Row &o) {
+    if constexpr (WC) return;
     const int slot = ring(kk);
     if (r < 2) {
       vec v;
@@ -393,10 +484,7 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
 
     // ---- P1: H1(k)
     if (doH1) {
-      const S iax = rowv(0, rk), Lz = plv(0, k);
-      S c0y[V], Lx[V];
-      ldsv(cyv(0, rk), c0y);
-      ldsv(sX + ln * V, Lx);
+      const Metric o = metric(0, rk, k);
       S EX[V], EY[V + 1], EZ[V + 1];
 #pragma unroll
       for (int q = 0; q < V + 1; ++q) {
@@ -405,14 +493,13 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
       }
 #pragma unroll
       for (int q = 0; q < V; ++q) {
-        const S *t = sMat + NM * (int)((code >> (8 * q)) & 0xffu);
-        const S a0 = (S)(iax * t[0]), a1 = (S)(c0y[q] * t[1]), a2 = (S)(iAz[0][q] * t[2]);
-        H1[0][q] = h_row<S, S, DESC>(h0[0][q], a0, dt, Ly, Lz, EY[q], Ek1[1][q], EZ[q],
-                                     e0(2, Pu, q), +1, -1);
-        H1[1][q] = h_row<S, S, DESC>(h0[1][q], a1, dt, Lx[q], Lz, EX[q], Ek1[0][q], EZ[q],
-                                     EZ[q + 1], -1, +1);
-        H1[2][q] = h_row<S, S, DESC>(h0[2][q], a2, dt, Lx[q], Ly, EX[q],
-                                     e0(0, Pu, q), EY[q], EY[q + 1], +1, -1);
+        S w[6];
+        h_w(trow(code, q), q, o, w);
+        H1[0][q] = t2_h<DESC>(h0[0][q], w[0], w[1], EY[q], Ek1[1][q], EZ[q], e0(2, Pu, q),
+                              +1, -1);
+        H1[1][q] = t2_h<DESC>(h0[1][q], w[2], w[3], EX[q], Ek1[0][q], EZ[q], EZ[q + 1], -1, +1);
+        H1[2][q] = t2_h<DESC>(h0[2][q], w[4], w[5], EX[q], e0(0, Pu, q), EY[q], EY[q + 1],
+                              +1, -1);
         h1(0, P, q) = H1[0][q];
         h1(2, P, q) = H1[2][q];
         if (q == V - 1) h1(1, P, q) = H1[1][q];
@@ -422,27 +509,25 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
 
     // ---- P2: E1(k), then H2(k-1)
     if (doE1) {
-      const S itax = rowv(1, rk), tLz = plv(1, k), bm = plv(2, k);
-      S c1y[V], tLx[V];
-      ldsv(cyv(1, rk), c1y);
-      ldsv(sX + (Q + ln) * V, tLx);
+      const S bm = plv(2, k);
+      const Metric o = metric(1, rk, k);
       const S HYm = h1(1, P - 1, V - 1), HZm = h1(2, P - 1, V - 1);  // -x neighbours
       S s2[V];
 #pragma unroll
       for (int q = 0; q < V; ++q) {
-        const S *t = sMat + NM * (int)((code >> (8 * q)) & 0xffu);
-        const S b0 = (S)(t[3] * itax), b1 = (S)(t[4] * c1y[q]), b2 = (S)(t[5] * itAz[0][q]);
-        S d0 = e_sum<S>(b0, tLy, tLz, H1p[1][q], H1[1][q], h1(2, Pd, q), H1[2][q], +1, -1);
-        S d1 = e_sum<S>(b1, tLx[q], tLz, H1p[0][q], H1[0][q], q ? H1[2][q - 1] : HZm, H1[2][q],
-                        -1, +1);
-        S d2 = e_sum<S>(b2, tLx[q], tLy, h1(0, Pd, q), H1[0][q], q ? H1[1][q - 1] : HYm,
-                        H1[1][q], +1, -1);
+        const S *t = trow(code, q);
+        S w[6];
+        e_w(t, q, o, w);
+        S d0 = t2_e(w[0], w[1], H1p[1][q], H1[1][q], h1(2, Pd, q), H1[2][q], +1, -1);
+        S d1 = t2_e(w[2], w[3], H1p[0][q], H1[0][q], q ? H1[2][q - 1] : HZm, H1[2][q], -1, +1);
+        S d2 = t2_e(w[4], w[5], h1(0, Pd, q), H1[0][q], q ? H1[1][q - 1] : HYm, H1[1][q],
+                    +1, -1);
         s2[q] = d2;
         const S o0 = e0(0, P, q), o1 = e0(1, P, q), o2 = e0(2, P, q);  // E0(k) as staged
         if (COND) {  // J = sigma E0
-          d0 = d0 - t[3] * (S)(t[6] * o0);
-          d1 = d1 - t[4] * (S)(t[7] * o1);
-          d2 = d2 - t[5] * (S)(t[8] * o2);
+          d0 = d0 - t[IE] * (S)(t[SG] * o0);
+          d1 = d1 - t[IE + 1] * (S)(t[SG + 1] * o1);
+          d2 = d2 - t[IE + 2] * (S)(t[SG + 2] * o2);
         }
         E1[0][q] = (S)(o0 + dt * d0);
         E1[1][q] = (S)(o1 + dt * d1);
@@ -451,8 +536,7 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
       if (qbeam >= 0) {  // the beam's current instead on its line
 #pragma unroll
         for (int q = 0; q < V; ++q) {
-          const S *t = sMat + NM * (int)((code >> (8 * q)) & 0xffu);
-          const S d2 = s2[q] - t[5] * bm;
+          const S d2 = s2[q] - trow(code, q)[IE + 2] * bm;
           if (q == qbeam) E1[2][q] = (S)(e0(2, P, q) + dt * d2);
         }
       }
@@ -462,10 +546,7 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
         buf_st<RAG>(buf_of(E1out, 3 * NB), ofs, (I)k * sz * ES, NB, E1);
     }
     if (doH2 && p >= kstart) {  // H2 below plane 0 stays 0
-      const S iaxp = rowv(0, rp), Lzp = plv(0, p);
-      S c0yp[V], Lx[V];
-      ldsv(cyv(0, rp), c0yp);
-      ldsv(sX + ln * V, Lx);
+      const Metric o = metric(0, rp, p);
       // E1(p): own row from slot Pd (x neighbour at q = V), row j+1 from slot P
       S EX[V], EY[V + 1], EZ[V + 1];
 #pragma unroll
@@ -475,14 +556,12 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
       }
 #pragma unroll
       for (int q = 0; q < V; ++q) {
-        const S *t = sMat + NM * (int)((codep >> (8 * q)) & 0xffu);
-        const S a0 = (S)(iaxp * t[0]), a1 = (S)(c0yp[q] * t[1]), a2 = (S)(iAz[0][q] * t[2]);
-        H2[0][q] = h_row<S, S, DESC>(H1p[0][q], a0, dt, Ly, Lzp, EY[q], E1[1][q], EZ[q],
-                                     e1(2, P, q), +1, -1);
-        H2[1][q] = h_row<S, S, DESC>(H1p[1][q], a1, dt, Lx[q], Lzp, EX[q], E1[0][q], EZ[q],
-                                     EZ[q + 1], -1, +1);
-        H2[2][q] = h_row<S, S, DESC>(H1p[2][q], a2, dt, Lx[q], Ly, EX[q],
-                                     e1(0, P, q), EY[q], EY[q + 1], +1, -1);
+        S w[6];
+        h_w(trow(codep, q), q, o, w);
+        H2[0][q] = t2_h<DESC>(H1p[0][q], w[0], w[1], EY[q], E1[1][q], EZ[q], e1(2, P, q), +1, -1);
+        H2[1][q] = t2_h<DESC>(H1p[1][q], w[2], w[3], EX[q], E1[0][q], EZ[q], EZ[q + 1], -1, +1);
+        H2[2][q] = t2_h<DESC>(H1p[2][q], w[4], w[5], EX[q], e1(0, P, q), EY[q], EY[q + 1],
+                              +1, -1);
         h2(0, Pd, q) = H2[0][q];
         h2(2, Pd, q) = H2[2][q];
         if (q == V - 1) h2(1, Pd, q) = H2[1][q];
@@ -510,27 +589,25 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
     const uint32_t coden = load_code(kn);
     load_e(k < kend ? k + 2 : g.Nz, Ek1);
     if (own && l2e) {
-      const S itaxp = rowv(1, rp), tLzp = plv(1, p), bv2 = plv(3, p);
-      S c1yp[V], tLx[V];
-      ldsv(cyv(1, rp), c1yp);
-      ldsv(sX + (Q + ln) * V, tLx);
+      const S bv2 = plv(3, p);
+      const Metric o = metric(1, rp, p);
       const S HYm = h2(1, Pd - 1, V - 1), HZm = h2(2, Pd - 1, V - 1);
       S E2[3][V], s2[V], Jn[3][V];
 #pragma unroll
       for (int q = 0; q < V; ++q) {
-        const S *t = sMat + NM * (int)((codep >> (8 * q)) & 0xffu);
-        const S b0 = (S)(t[3] * itaxp), b1 = (S)(t[4] * c1yp[q]), b2 = (S)(t[5] * itAz[0][q]);
-        S d0 = e_sum<S>(b0, tLy, tLzp, H2p[1][q], H2[1][q], h2(2, Pdd, q), H2[2][q], +1, -1);
-        S d1 = e_sum<S>(b1, tLx[q], tLzp, H2p[0][q], H2[0][q], q ? H2[2][q - 1] : HZm, H2[2][q],
-                        -1, +1);
-        S d2 = e_sum<S>(b2, tLx[q], tLy, h2(0, Pdd, q), H2[0][q], q ? H2[1][q - 1] : HYm,
-                        H2[1][q], +1, -1);
+        const S *t = trow(codep, q);
+        S w[6];
+        e_w(t, q, o, w);
+        S d0 = t2_e(w[0], w[1], H2p[1][q], H2[1][q], h2(2, Pdd, q), H2[2][q], +1, -1);
+        S d1 = t2_e(w[2], w[3], H2p[0][q], H2[0][q], q ? H2[2][q - 1] : HZm, H2[2][q], -1, +1);
+        S d2 = t2_e(w[4], w[5], h2(0, Pdd, q), H2[0][q], q ? H2[1][q - 1] : HYm, H2[1][q],
+                    +1, -1);
         s2[q] = d2;
         const S o0 = e1(0, Pd, q), o1 = e1(1, Pd, q), o2 = e1(2, Pd, q);  // E1(k-1)
         if (COND) {
-          d0 = d0 - t[3] * (S)(t[6] * o0);
-          d1 = d1 - t[4] * (S)(t[7] * o1);
-          d2 = d2 - t[5] * (S)(t[8] * o2);
+          d0 = d0 - t[IE] * (S)(t[SG] * o0);
+          d1 = d1 - t[IE + 1] * (S)(t[SG + 1] * o1);
+          d2 = d2 - t[IE + 2] * (S)(t[SG + 2] * o2);
         }
         E2[0][q] = (S)(o0 + dt * d0);
         E2[1][q] = (S)(o1 + dt * d1);
@@ -539,8 +616,7 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
       if (qbeam >= 0) {
 #pragma unroll
         for (int q = 0; q < V; ++q) {
-          const S *t = sMat + NM * (int)((codep >> (8 * q)) & 0xffu);
-          const S d2 = s2[q] - t[5] * bv2;
+          const S d2 = s2[q] - trow(codep, q)[IE + 2] * bv2;
           if (q == qbeam) E2[2][q] = (S)(e1(2, Pd, q) + dt * d2);
         }
         if (!COND) J[2 * g.N + (int64_t)p * g.sz + cell + qbeam] = bv2;
@@ -551,9 +627,9 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
         const Buf bJ = buf_of(J, 3 * NB);
 #pragma unroll
         for (int q = 0; q < V; ++q) {
-          const S *t = sMat + NM * (int)((codep >> (8 * q)) & 0xffu);
+          const S *t = trow(codep, q);
 #pragma unroll
-          for (int c = 0; c < 3; ++c) Jn[c][q] = (S)(t[6 + c] * E2[c][q]);
+          for (int c = 0; c < 3; ++c) Jn[c][q] = (S)(t[SG + c] * E2[c][q]);
         }
         buf_st<RAG>(bJ, ofs, (I)p * sz * ES, NB, Jn);
       }
@@ -575,24 +651,24 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
   }
 }
 
-template <typename S, bool COND, bool DESC, bool RAG>
+template <typename S, bool COND, bool DESC, bool RAG, bool WC>
 __global__ void __launch_bounds__(T2_NT)
 k_fused4_t2(GridDev g, MetricDev<S> m, const S *__restrict__ Ein, const S *__restrict__ Hin,
             S *__restrict__ Eout, S *__restrict__ Hout, S *__restrict__ J, Coefs<S> cf, S dt,
             T2Aux x, const S *__restrict__ beam1, const S *__restrict__ beam2,
             S *__restrict__ cap) {
-  t2_tile<S, COND, DESC, RAG>(g, m, Ein, Hin, Eout, Hout, J, cf, dt, x, beam1, beam2, cap,
+  t2_tile<S, COND, DESC, RAG, WC>(g, m, Ein, Hin, Eout, Hout, J, cf, dt, x, beam1, beam2, cap,
                              xcd_tile(blockIdx.x, x.ntx * x.nty * x.ntz));
 }
 
 // The same, the E of the first step stored too (E1out).
-template <typename S, bool COND, bool DESC, bool RAG>
+template <typename S, bool COND, bool DESC, bool RAG, bool WC>
 __global__ void __launch_bounds__(T2_NT)
 k_fused4_t2_mon(GridDev g, MetricDev<S> m, const S *__restrict__ Ein, const S *__restrict__ Hin,
                 S *__restrict__ Eout, S *__restrict__ Hout, S *__restrict__ J, Coefs<S> cf, S dt,
                 T2Aux x, const S *__restrict__ beam1, const S *__restrict__ beam2,
                 S *__restrict__ cap, S *__restrict__ E1out) {
-  t2_tile<S, COND, DESC, RAG, true>(g, m, Ein, Hin, Eout, Hout, J, cf, dt, x, beam1, beam2, cap,
+  t2_tile<S, COND, DESC, RAG, WC, true>(g, m, Ein, Hin, Eout, Hout, J, cf, dt, x, beam1, beam2, cap,
                                     xcd_tile(blockIdx.x, x.ntx * x.nty * x.ntz), E1out);
 }
 
@@ -609,7 +685,7 @@ struct T2Batch {
 // its share of the CUs, one workgroup each. 24 grids of 28 to 160 cells a side
 // (5.3 million cells), FP32: about 100 us per launch, 50 a step, against 92 + 4.5
 // of the one-step kernel and its step counter.
-template <typename S, bool COND, bool DESC, bool RAG>
+template <typename S, bool COND, bool DESC, bool RAG, bool WC>
 __global__ void __launch_bounds__(T2_NT)
 k_fused4_t2_batch(const T2Batch<S> *__restrict__ d, int ninst, int ntiles, int s, int step0,
                   int end, int flip) {
@@ -629,7 +705,7 @@ k_fused4_t2_batch(const T2Batch<S> *__restrict__ d, int ninst, int ntiles, int s
   const MetricDev<S> m = e.b.m;
   const Coefs<S> cf = e.b.cf;
   const S *row = e.b.beam_table + (e.b.beam_row0 + s) * g.Nz;
-  t2_tile<S, COND, DESC, RAG>(g, m, flip ? e.b.E2 : e.b.E, flip ? e.b.H2 : e.b.H,
+  t2_tile<S, COND, DESC, RAG, WC>(g, m, flip ? e.b.E2 : e.b.E, flip ? e.b.H2 : e.b.H,
                               flip ? e.b.E : e.b.E2, flip ? e.b.H : e.b.H2, e.b.J, cf, e.b.dt, x,
                               row, row + g.Nz, e.b.cap, tile - e.tile0);
 }

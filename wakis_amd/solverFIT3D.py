@@ -213,6 +213,8 @@ class SolverFIT3D(RoutinesMixin):
         self.code_escape_max = 0.05
         self._code_escape = False
         self._lut_key = None
+        self.use_weight_codes = True
+        self._wkey = self._wcode = self._wtab = None
         self._code = self._mat = self._metric2d = None
         self._nmat = 0
         self.update_tensors("all", _initial=True)
@@ -577,6 +579,42 @@ class SolverFIT3D(RoutinesMixin):
         self._code_escape = esc is not None
         return True
 
+    def _weight_table(self):
+        """Weight codes for the two-step kernel (wf_step_args.wcode): per cell a
+        row of the products of metric, material and dt, where the metric is
+        uniform along each axis but for its first and last cells and at most 255
+        distinct rows occur. Valid as long as the material codes and dt."""
+        key = (self._lut_key, float(self.dt))
+        if key == self._wkey:
+            return self._wcode is not None
+        self._wkey, self._wcode, self._wtab = key, None, None
+        n, nk = _lib.WF_WEIGHT_ROW, 27 * self._nmat
+        buf = torch.empty(nk * n + nk + 1, dtype=torch.int32, device=self.device)
+        lib, st = _lib.lib(), _lib.stream_ptr()
+        _lib.check(lib.wf_weight_rows(
+            self._handle, _lib.ptr(self._code), _lib.ptr(self._mat), self._nmat,
+            _lib.ptr(self._metric2d), float(self.dt), _lib.ptr(buf), _lib.ptr(buf[nk * n:]), st),
+            "wf_weight_rows")
+        host = buf.cpu().numpy()
+        rows, used = host[:nk * n].reshape(nk, n), host[nk * n:]
+        if used[nk]:
+            return False
+        sel = np.flatnonzero(used[:nk])
+        distinct, inv = np.unique(rows[sel], axis=0, return_inverse=True)
+        if len(distinct) > 255:
+            return False
+        table = np.zeros((len(distinct) + 1, n), dtype=np.int32)  # row 0: cells off the grid
+        table[1:] = distinct
+        row_of = np.zeros(nk, dtype=np.uint8)
+        row_of[sel] = 1 + inv.reshape(-1)
+        row_of = torch.as_tensor(row_of, device=self.device)
+        self._wcode = torch.empty(self.N, dtype=torch.uint8, device=self.device)
+        self._wtab = torch.as_tensor(table.view(np.float32), device=self.device)
+        _lib.check(lib.wf_weight_codes(self._handle, _lib.ptr(self._code), self._nmat,
+                                       _lib.ptr(row_of), _lib.ptr(self._wcode), st),
+                   "wf_weight_codes")
+        return True
+
     def _masked_zero(self):
         """True if E is zero on every PEC-masked edge, H on every PMC-masked
         face, and the beam line is not on a masked edge.
@@ -713,6 +751,14 @@ class SolverFIT3D(RoutinesMixin):
                                                   _lib.ptr(self._metric2d))
             args.nmat = self._nmat
             args.code_escape = int(self._code_escape)
+            # weight codes where pairs of steps run: built by the first longer call
+            # (100 to 200 us, a few steps' gain at any size), then kept
+            if (self.use_weight_codes and args.two_step and args.beam_table and args.zero_masked
+                    and self.dtype == np.float32 and not self._code_escape
+                    and (args.nsteps >= 64 or self._wkey is not None)
+                    and self._weight_table()):
+                args.wcode, args.wtab = _lib.ptr(self._wcode), _lib.ptr(self._wtab)
+                args.nw = self._wtab.shape[0]
         if args.jmode == _lib.WF_J_FULL and not args.conductive:
             raise RuntimeError("internal: fused path without a J mode")
         if args.conductive:
