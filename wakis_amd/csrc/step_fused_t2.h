@@ -26,15 +26,19 @@
 // consecutive words (a gap between the rows of a wave cost a second pass of
 // every access). Rows of exactly whole waves keep the gap instead of the lane.
 //
-// Per plane, with one barrier after each phase:
-//   P1 H1(k) on rows 0..T+2; stage H1(k)
+// Per plane, with a barrier after P1 and one after P2:
+//   P1 H1(k) on rows 0..T+2; stage H1(k); issue the loads of H0(k+1) and of the
+//      metric rows of plane k+1
 //   P2 E1(k) on rows 1..T+2; H2(k-1) on rows 1..T+1 (reads E1(k-1) staged in
-//      the previous P3); stage H2(k-1)
-//   P3 stage E0(k+1); issue the loads of E0(k+2), of the codes of plane k+1
-//      and of its metric rows; E2(k-1) on rows 2..T+1, stores; stage E1(k)
-//      and the metric rows; issue the loads of H0(k+1)
-// Loads are in flight during the E2 update before their use, no register is
-// copied from a load before that use, and the per-plane scalars (Lz, tLz, the
+//      the previous P3); stage H2(k-1), E0(k+1) and the metric rows; issue the
+//      loads of E0(k+2) and of the codes of plane k+1
+//   P3 E2(k-1) on rows 2..T+1, stores; stage E1(k)
+// P3 and the next P1 touch different buffers and need no barrier between them.
+// The loads of H0 are in flight over a plane, those of E0 over P3 (issued with
+// E0's, H0 cost 641 / 596 ms a pass at 256x256x512 FP32, 172 / 153 with
+// conduction at 200x200x400, 93 / 83 at 160x160x200 FP64; E0 a plane earlier,
+// in 12 more registers, gave nothing). No register is
+// copied from a load before its use, and the per-plane scalars (Lz, tLz, the
 // beam) are staged in LDS once per launch, so the waves rarely wait for
 // memory. LDS holds one block per component and cell of a lane, rows end to
 // end in it, so a single-word read takes consecutive words in consecutive
@@ -505,6 +509,10 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
         if (q == V - 1) h1(1, P, q) = H1[1][q];
       }
     }
+    const int kn = k < kend ? k + 1 : g.Nz;  // nothing is read after the last plane
+    Row row;
+    load_row(kn, row);
+    load_h(kn, h0);
     __syncthreads();
 
     // ---- P2: E1(k), then H2(k-1)
@@ -573,21 +581,28 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
     for (int c = 0; c < 3; ++c)
 #pragma unroll
       for (int q = 0; q < V; ++q) H1p[c][q] = H1[c][q];
-    __syncthreads();
-
-    // ---- P3: stage E0(k+1) (sE0 is free once E1(k) is done); loads of plane
-    // k+1 and of E0(k+2); E2(k-1) on the own rows, stores; stage E1(k)
+    // stage E0(k+1): other lanes read this lane's slots in P1 only
     if (act) {
 #pragma unroll
       for (int c = 0; c < 3; ++c)
 #pragma unroll
         for (int q = 0; q < V; ++q) e0(c, P, q) = Ek1[c][q];
     }
-    const int kn = k < kend ? k + 1 : g.Nz;  // nothing is read after the last plane
-    Row row;
-    load_row(kn, row);
-    const uint32_t coden = load_code(kn);
-    load_e(k < kend ? k + 2 : g.Nz, Ek1);
+    put_row(k + 1, row);
+    // the loads of E0(k+2) before the barrier, FP64 after it (ms a pass: 91x75x161
+    // FP32 16.4 against 16.5, 300x220x180 72.4 / 73.7, 160x160x200 FP64 85.2 / 82.6)
+    constexpr bool LATE = sizeof(S) == 8;
+    uint32_t coden;
+    const auto loads = [&]() {
+      coden = load_code(kn);
+      load_e(k < kend ? k + 2 : g.Nz, Ek1);
+    };
+    if (!LATE) loads();
+    __syncthreads();
+
+    // ---- P3: E2(k-1) on the own rows, stores; stage E1(k). No barrier before
+    // the next P1, which reads E0(k+1) and writes H1(k+1) only
+    if (LATE) loads();
     if (own && l2e) {
       const S bv2 = plv(3, p);
       const Metric o = metric(1, rp, p);
@@ -642,12 +657,9 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
 #pragma unroll
         for (int q = 0; q < V; ++q) e1(c, Pd, q) = E1[c][q];
     }
-    put_row(k + 1, row);
-    load_h(kn, h0);
     // level 2 of the next plane uses this plane's coefficients
     codep = code;
     code = coden;
-    __syncthreads();
   }
 }
 
