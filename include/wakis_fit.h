@@ -65,6 +65,14 @@ typedef struct wf_grid {
   const double *tLx, *tLy, *tLz; /* host, dual edge lengths after periodic/ABC edits */
 } wf_grid;
 
+/* A value written to one component of E or H on the cells [lo, hi) before each
+ * step of a call. values: host array of one value per step, rounded to the
+ * storage type; NULL: none. */
+typedef struct {
+  const double *values;
+  int32_t comp, lo[3], hi[3];
+} wf_box_source;
+
 /* One leapfrog batch. Replaces SolverFIT3D._one_step (solverFIT3D.py:482-503)
  * called nsteps times, plus Beam.update's J line write (sources.py:108-110) and
  * wakesolve's per-step Ez window save (routines.py:419-425, 440).
@@ -200,6 +208,11 @@ typedef struct wf_step_args {
   const void *wcode;      /* device uint8[N]                                          */
   const void *wtab;       /* device FP32 [nw][WF_WEIGHT_ROW]                          */
   int32_t nw;             /* 1..256                                                   */
+  /* Path 0, optional: what emsolve does around its steps. Sources written before
+   * each step, and wf_abc_low of these faces after it. Not with captures,
+   * trajectories or monitors, not in batches. */
+  wf_box_source src_E, src_H;
+  int32_t abc_low;
 } wf_step_args;
 
 /* Values of a row of the weight table: the 6 weights of the H rows, the 6 of

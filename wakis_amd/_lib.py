@@ -25,6 +25,11 @@ class WfGrid(ctypes.Structure):
     ]
 
 
+class WfBoxSource(ctypes.Structure):
+    _fields_ = [("values", POINTER(c_double)), ("comp", c_int32), ("lo", c_int32 * 3),
+                ("hi", c_int32 * 3)]
+
+
 class WfStepArgs(ctypes.Structure):
     _fields_ = [
         ("E", c_void_p), ("H", c_void_p), ("J", c_void_p),
@@ -48,6 +53,7 @@ class WfStepArgs(ctypes.Structure):
         ("mon_nf", c_int32), ("mon_phase_f32", c_int32), ("two_step", c_int32),
         ("two_step_used", c_int32), ("mon_work", c_void_p), ("mon_slots", c_int32),
         ("wcode", c_void_p), ("wtab", c_void_p), ("nw", c_int32),
+        ("src_E", WfBoxSource), ("src_H", WfBoxSource), ("abc_low", c_int32),
     ]
 
 

@@ -196,23 +196,47 @@ int step_general(wf_handle *h, const wf_step_args *a, const wf::MetricDev<S> &m,
   x.cap_ix0 = a->cap_ix0; x.cap_iy0 = a->cap_iy0; x.cap_nx = a->cap_nx; x.cap_ny = a->cap_ny;
   x.cap_samples = a->cap_samples;
   const Cm dt = (Cm)a->dt;
+  // sources: that of E is written by the E sweep of the step before, unless the
+  // low-face copies come between; that of H by the step's own H sweep
+  const auto source = [&](const wf_box_source &b, int s) {
+    wf::BoxSource<S> o{};
+    o.comp = b.values ? b.comp : -1;
+    for (int d = 0; d < 3; ++d) { o.lo[d] = b.lo[d]; o.hi[d] = b.hi[d]; }
+    if (b.values) o.v = (S)b.values[s];
+    return o;
+  };
+  const wf::BoxSource<S> none = source(wf_box_source{}, 0);
   for (int s = 0; s < a->nsteps; ++s) {
+    if (a->src_E.values && (s == 0 || a->abc_low)) {
+      const wf::BoxSource<S> b = source(a->src_E, s);
+      const dim3 gb((unsigned)((b.hi[0] - b.lo[0] + wf::EX_TX - 1) / wf::EX_TX),
+                    (unsigned)((b.hi[1] - b.lo[1] + wf::EX_TY - 1) / wf::EX_TY),
+                    (unsigned)std::min(b.hi[2] - b.lo[2], 65535));
+      hipLaunchKernelGGL(wf::k_box_source<S>, gb, blk, 0, st, g, b, (S *)a->E);
+      WF_LAUNCH_CHECK();
+    }
     hipLaunchKernelGGL((wf::k_h_exact<S, Cm>), grd, blk, 0, st, g, m, (S *)a->H,
-                       (const S *)a->E, (const S *)a->a, dt);
+                       (const S *)a->E, (const S *)a->a, dt, source(a->src_H, s));
     WF_LAUNCH_CHECK();
+    const bool ahead = a->src_E.values && !a->abc_low && s + 1 < a->nsteps;
+    const wf::BoxSource<S> es = ahead ? source(a->src_E, s + 1) : none;
     const S *row = a->beam_table ? (const S *)a->beam_table + (a->beam_row0 + s) * g.Nz : nullptr;
     x.cap_sample = a->cap_sample0 + s;
     S *cap = (S *)a->capture;
 #define WF_E_LAUNCH(JM, CO)                                                                  \
   hipLaunchKernelGGL((wf::k_e_exact<S, Cm, JM, CO>), grd, blk, 0, st, g, m,                \
                      (S *)a->E, (const S *)a->H, (S *)a->J, (const S *)a->b,                 \
-                     (const S *)a->ieps, (const S *)a->sigma, dt, x, row, cap)
+                     (const S *)a->ieps, (const S *)a->sigma, dt, x, row, cap, es)
     if (a->conductive) WF_E_LAUNCH(2, true);
     else if (a->jmode == WF_J_FULL) WF_E_LAUNCH(2, false);
     else if (a->jmode == WF_J_LINE) WF_E_LAUNCH(1, false);
     else WF_E_LAUNCH(0, false);
 #undef WF_E_LAUNCH
     WF_LAUNCH_CHECK();
+    if (a->abc_low) {
+      const int rc = wf_abc_low(h, a->E, a->H, a->abc_low, st);
+      if (rc != WF_OK) return rc;
+    }
     if (a->traj_E) {
       traj_store<S>(h, a, (const S *)a->E, (const S *)a->H, a->traj_slot0 + s + 1, st);
       WF_LAUNCH_CHECK();
@@ -316,6 +340,22 @@ int check_step_args(const wf_handle *h, const wf_step_args *a, const char *who) 
                      (a->mon_phase_f32 != 0 && a->mon_phase_f32 != 1)))
     return fail(WF_EINVAL, "%s: the field monitor needs a phase table, mon_nf >= 1, "
                 "mon_row0 >= 0 and mon_phase_f32 0 or 1", who);
+  if (a->src_E.values || a->src_H.values || a->abc_low) {
+    if (a->path != 0 || a->traj_E || a->mon_acc || a->capture || a->abc_low < 0 ||
+        a->abc_low > 7)
+      return fail(WF_EINVAL, "%s: box sources and low-face copies go with path 0 and without "
+                  "captures", who);
+    const int n[3] = {h->g.Nx, h->g.Ny, h->g.Nz};
+    for (const wf_box_source *b : {&a->src_E, &a->src_H}) {
+      if (!b->values) continue;
+      if (b->comp < 0 || b->comp > 2) return fail(WF_EINVAL, "%s: bad source component", who);
+      for (int d = 0; d < 3; ++d)
+        if (b->lo[d] < 0 || b->hi[d] > n[d] || b->lo[d] >= b->hi[d])
+          return fail(WF_ERANGE, "%s: source box outside the grid", who);
+      if ((b->hi[1] - b->lo[1] + wf::EX_TY - 1) / wf::EX_TY > 65535)
+        return fail(WF_ERANGE, "%s: source box too large", who);
+    }
+  }
   if (a->wcode && (!a->wtab || a->nw < 1 || a->nw > 256))
     return fail(WF_EINVAL, "%s: weight codes need a table of 1..256 rows", who);
   if (a->mon_slots < 0) return fail(WF_EINVAL, "%s: mon_slots < 0", who);

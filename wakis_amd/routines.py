@@ -8,6 +8,7 @@ inside the same step calls. There is no per-step host traffic unless a
 callback asks for it.
 """
 
+import ctypes
 import os
 import time
 
@@ -73,7 +74,10 @@ class RoutinesMixin:
 
     def _emsolve_loop(self, Nt, source, callback, hfs, save_every, sub, low_abc):
         xx, yy, zz = sub
-        for n in range(Nt):
+        n0 = 0  # steps taken: the first and the last below, the others in one go where they can
+        if Nt > 3 and callback is None and not hfs:
+            n0 = self._emsolve_source_steps(Nt, source, low_abc)
+        for n in range(n0, Nt):
             if source is not None:
                 source.update(self, n * self.dt)
             if hfs and n % save_every == 0:
@@ -86,6 +90,50 @@ class RoutinesMixin:
                                                  _lib.stream_ptr()), "wf_abc_low")
             if callback is not None:
                 callback(self, n * self.dt)
+
+    def _emsolve_source_steps(self, Nt, source, low_abc):
+        """Steps 0 .. Nt-2 of an emsolve with a plane wave, the source and the
+        low-face copies inside the library's step loop; returns the number of
+        steps taken (0: none). For runs whose every step takes the exact general
+        path: a conductive grid (a write to E ends J = sigma E) or one whose
+        flat-index wrap terms couple live cells whatever the fields hold."""
+        from .sources import PlaneWave
+        if type(source) is not PlaneWave or "update" in vars(source):
+            return 0
+        if self.path == "fused" or self.keep_previous_fields or not (
+                self.path == "general" or self.use_conductivity
+                or self._jmode() == _lib.WF_J_FULL or self._compute_f64()
+                or self._wraps_live()):
+            return 0
+        # the first step sets the source up and clears the ghosts
+        source.update(self, 0 * self.dt)
+        self.one_step()
+        abc = low_abc if self.activate_abc else 0
+        if abc:
+            _lib.check(_lib.lib().wf_abc_low(self._handle, _lib.ptr(self.E.array),
+                                             _lib.ptr(self.H.array), abc, _lib.stream_ptr()),
+                       "wf_abc_low")
+        box = source._box(self)
+        if box is None or any(np.ndim(v) for v in source._values(self.dt)):
+            return 1
+        n, size = 1, 32  # the host evaluates a chunk while the GPU runs the one before
+        while n < Nt - 1:
+            k = min(size, Nt - 1 - n)
+            val = np.array([[float(v) for v in source._values(i * self.dt)]
+                            for i in range(n, n + k)]).T.copy()
+            self.E.version += k
+            self.H.version += k
+            args = self._step_args(k)
+            args.abc_low = abc
+            for src, comp, v in ((args.src_H, 1, val[0]), (args.src_E, 0, val[1])):
+                src.values = v.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+                src.comp, src.lo[:], src.hi[:] = comp, box[0], box[1]
+            _lib.check(_lib.lib().wf_step(self._handle, ctypes.byref(args), _lib.stream_ptr()),
+                       "wf_step")
+            self._finish_run(False, False)
+            self.nstep += k
+            n += k
+        return n
 
     def wakesolve(self, wakelength, wake=None, callback=None, compute_plane="both", plot=False,
                   plot_func=None, plot_from=None, plot_every=1, plot_until=None, save_J=False,

@@ -213,6 +213,7 @@ class SolverFIT3D(RoutinesMixin):
         self.code_escape_max = 0.05
         self._code_escape = False
         self._lut_key = None
+        self._wlive_key = None
         self.use_weight_codes = True
         self._wkey = self._wcode = self._wtab = None
         self._code = self._mat = self._metric2d = None
@@ -657,14 +658,25 @@ class SolverFIT3D(RoutinesMixin):
                self._beam_line)
         if key == self._wrap_key:
             return self._wrap_ok
-        self._wrap_key, self._wrap_ok = key, self._wraps_dead_now()
+        live = self._wlive_key == self._fold_count and self._wlive
+        self._wrap_key, self._wrap_ok = key, not live and self._wraps_dead_now()
+        if not self._wrap_ok:
+            self._wraps_live()  # live for good: the next write to a field asks no more
         return self._wrap_ok
 
-    def _wraps_dead_now(self):
+    def _wraps_live(self):
+        """True if a wrap term acts on a column with a coefficient: then it is not
+        dead whatever the fields hold. Valid until coefficients are re-folded."""
+        if self._wlive_key != self._fold_count:
+            self._wlive_key, self._wlive = self._fold_count, not self._wraps_dead_now(False)
+        return self._wlive
+
+    def _wraps_dead_now(self, fields=True):
         """The test of ``_wraps_dead`` on the boundary planes. Each wrap term
         pairs a row with the column one flat index away (+-1 across a row end,
         +-Nx across the last row of a plane), so rows and columns are two views
-        of the same boundary plane shifted by one element."""
+        of the same boundary plane shifted by one element. ``fields`` False:
+        every column without a coefficient counts as frozen."""
         Nx, Ny, Nz = self.Nx, self.Ny, self.Nz
         dev = self.device
         a3 = self._a.view(3, Nz, Ny, Nx)
@@ -685,12 +697,16 @@ class SolverFIT3D(RoutinesMixin):
             return face_mask_kji(c, zbits, Nx, Ny, Nz, dev)
 
         def frozen_E(c, sl):  # E column frozen at zero (no coefficient, no source)
+            if not fields:
+                return b3[c][sl] == 0
             fz = (b3[c][sl] == 0) & (E3[c][sl] == 0) & ((ie3[c][sl] == 0) | (J3[c][sl] == 0))
             if beam is not None and c == 2:
                 fz = fz & ~beam[sl]
             return fz
 
         def frozen_H(c, sl):
+            if not fields:
+                return a3[c][sl] == 0
             return (a3[c][sl] == 0) & (H3[c][sl] == 0)
 
         tL = [torch.as_tensor(self._tL1[0], device=dev).view(1, 1, Nx).expand(Nz, Ny, Nx),

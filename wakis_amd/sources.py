@@ -94,14 +94,35 @@ class PlaneWave:
             if self.ys is None:
                 self.ys = slice(0, solver.Ny)
             self.is_first_update = False
+        hy, ex = self._values(t)
+        solver.H[self.xs, self.ys, self.zs, "y"] = hy
+        solver.E[self.xs, self.ys, self.zs, "x"] = ex
+
+    def _values(self, t):
+        """(H_y, E_x) on the plane at time t."""
         if t <= self.tmax:
-            solver.H[self.xs, self.ys, self.zs, "y"] = -self.amplitude * np.cos(
-                self.w * t + self.phase)
-            solver.E[self.xs, self.ys, self.zs, "x"] = (
-                self.amplitude * np.cos(self.w * t + self.phase) / (self.kz / (mu_0 * self.vp)))
-        else:
-            solver.H[self.xs, self.ys, self.zs, "y"] = 0.0
-            solver.E[self.xs, self.ys, self.zs, "x"] = 0.0
+            return (-self.amplitude * np.cos(self.w * t + self.phase),
+                    self.amplitude * np.cos(self.w * t + self.phase) / (self.kz / (mu_0 * self.vp)))
+        return 0.0, 0.0
+
+    def _box(self, solver):
+        """(lo, hi) of the plane's cells, or None if they are no box of the grid."""
+        lo, hi = [], []
+        for s, n in zip((self.xs, self.ys, self.zs), (solver.Nx, solver.Ny, solver.Nz)):
+            if isinstance(s, slice):
+                a, b, step = s.indices(n)
+                if step != 1:
+                    return None
+            elif isinstance(s, (int, np.integer)) and not isinstance(s, bool) and -n <= s < n:
+                a = int(s) % n
+                b = a + 1
+            else:
+                return None
+            if a >= b:
+                return None
+            lo.append(a)
+            hi.append(b)
+        return lo, hi
 
 
 class WavePacket:
