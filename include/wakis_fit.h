@@ -226,6 +226,11 @@ const char *wf_last_error(void);
 int wf_create(const wf_grid *g, wf_handle **out);
 int wf_destroy(wf_handle *h);
 
+/* Component comp (0..2) of F on the z line (ix, iy): Nz values from host memory,
+ * rounded to the storage type. Does not wait for the stream. */
+int wf_write_line(wf_handle *h, void *F, int32_t comp, int32_t ix, int32_t iy,
+                  const double *values, void *stream);
+
 /* Weights of the cells of a grid on FP32 material codes whose metric is the
  * same for all cells of a class: the first, the inner and the last cells of an
  * axis (uniform spacing). For class c = cx + 3 (cy + 3 cz) and material code m,

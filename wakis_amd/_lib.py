@@ -92,6 +92,8 @@ EXPORTS = {
     "wf_last_error": (ctypes.c_char_p, []),
     "wf_create": (c_int32, [POINTER(WfGrid), POINTER(c_void_p)]),
     "wf_destroy": (c_int32, [c_void_p]),
+    "wf_write_line": (c_int32, [c_void_p, c_void_p, c_int32, c_int32, c_int32, c_void_p,
+                                c_void_p]),
     "wf_weight_rows": (c_int32, [c_void_p, c_void_p, c_void_p, c_int32, c_void_p, c_double,
                                  c_void_p, c_void_p, c_void_p]),
     "wf_weight_codes": (c_int32, [c_void_p, c_void_p, c_int32, c_void_p, c_void_p, c_void_p]),

@@ -133,6 +133,30 @@ int wf_destroy(wf_handle *h) {
   return WF_OK;
 }
 
+int wf_write_line(wf_handle *h, void *F, int32_t comp, int32_t ix, int32_t iy,
+                  const double *values, void *stream) {
+  if (!h || !F || !values) return fail(WF_EINVAL, "wf_write_line: null argument");
+  if (comp < 0 || comp > 2) return fail(WF_EINVAL, "wf_write_line: bad component");
+  if (ix < 0 || ix >= h->g.Nx || iy < 0 || iy >= h->g.Ny)
+    return fail(WF_ERANGE, "wf_write_line: line (%d,%d) outside the grid", ix, iy);
+  const int64_t at = comp * h->g.N + ix + h->g.sy * iy;
+  const auto run = [&](auto zero) {
+    using S = decltype(zero);
+    wf::LineValues<S> l;
+    const int per = (int)(sizeof(l.v) / sizeof(S));
+    for (int k = 0; k < h->g.Nz; k += per) {
+      const int n = std::min(per, h->g.Nz - k);
+      for (int t = 0; t < n; ++t) l.v[t] = (S)values[k + t];
+      for (int t = n; t < per; ++t) l.v[t] = S(0);
+      hipLaunchKernelGGL(wf::k_write_line<S>, dim3(1), dim3(256), 0, (hipStream_t)stream,
+                         (S *)F + at + k * h->g.sz, h->g.sz, n, l);
+      WF_LAUNCH_CHECK();
+    }
+    return (int)WF_OK;
+  };
+  return h->dtype == WF_F64 ? run(0.0) : run(0.0f);
+}
+
 int wf_weight_rows(wf_handle *h, const void *code, const void *mat, int32_t nmat,
                    const void *metric2d, double dt, void *rows, int32_t *used, void *stream) {
   if (!h || !code || !mat || !metric2d || !rows || !used)

@@ -89,6 +89,19 @@ __device__ __forceinline__ void add_e_term(S &acc, S w, S v, bool ok, int sign) 
   acc = (sign > 0) ? acc + p : acc - p;
 }
 
+// Values of a z line in the kernel's arguments: no copy to the device, and no
+// wait for the stream as for one from pageable memory (a beam's line written from
+// Python and one step at 40x40x64 FP32: 49 against 26 us a step).
+template <typename S>
+struct LineValues {
+  S v[3072 / sizeof(S)];
+};
+template <typename S>
+__global__ void __launch_bounds__(256)
+k_write_line(S *__restrict__ F, int64_t stride, int n, LineValues<S> l) {
+  for (int t = threadIdx.x; t < n; t += 256) F[t * stride] = l.v[t];
+}
+
 // A value written to one component of a field on a box of cells before a step
 // (a plane source): the sweeps write it themselves, so it costs no launch. 240
 // steps at 64x64x60 FP32, source written by two fills from Python per step

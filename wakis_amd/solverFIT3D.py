@@ -449,7 +449,15 @@ class SolverFIT3D(RoutinesMixin):
         """J[ixs, iys, :, 'z'] = values without marking J as user-written."""
         line = (int(ixs), int(iys))
         v = self.J.version
-        self.J[ixs, iys, :, "z"] = values
+        if (type(values) is np.ndarray and values.dtype == np.float64
+                and values.shape == (self.Nz,) and 0 <= ixs < self.Nx and 0 <= iys < self.Ny):
+            values = np.ascontiguousarray(values)
+            _lib.check(_lib.lib().wf_write_line(self._handle, _lib.ptr(self.J.array), 2, line[0],
+                                                line[1], values.ctypes.data, _lib.stream_ptr()),
+                       "wf_write_line")
+            self.J.version += 1
+        else:
+            self.J[ixs, iys, :, "z"] = values
         if self._beam_line is None or self._beam_line == line:
             self.J.version = v  # J stays zero outside this one line
             if v == self._J_clean_version:
