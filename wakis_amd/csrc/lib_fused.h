@@ -57,7 +57,7 @@ template <typename S, int TY, int V, bool FR, bool WIDE>
 int step_fused4(wf_handle *h, wf_step_args *a, const wf::MetricDev<S> &m, hipStream_t st,
                 int fr_rows = 0) {
   const wf::GridDev &g = h->g;
-  wf::FusedAux x;
+  wf::FusedAux x{};
   x.ixs = (a->jmode == WF_J_LINE || a->beam_table || a->conductive) ? a->ixs : -1;
   x.iys = (x.ixs >= 0) ? a->iys : -1;
   x.cap_ix0 = a->cap_ix0; x.cap_iy0 = a->cap_iy0; x.cap_nx = a->cap_nx; x.cap_ny = a->cap_ny;
@@ -136,16 +136,25 @@ int step_fused4(wf_handle *h, wf_step_args *a, const wf::MetricDev<S> &m, hipStr
     cf.iAx = t; cf.iAy = t + yz; cf.iAz = t + yz + xz;
     cf.itAx = t + yz + xz + xy; cf.itAy = cf.itAx + yz; cf.itAz = cf.itAy + xz;
   }
+  // escape kernels fill the trajectory themselves
+  const bool traj_in = !WIDE && lut && a->code_escape && a->traj_E;
+  for (int d = 0; d < 3; ++d) { x.tlo[d] = a->traj_lo[d]; x.thi[d] = a->traj_hi[d]; }
   int cur = 0;
   for (int s = 0; s < a->nsteps; ++s) {
     const S *row = a->beam_table ? (const S *)a->beam_table + (a->beam_row0 + s) * g.Nz : nullptr;
     x.cap_sample = a->cap_sample0 + s;
     x.skip_j = (s + 1 < a->nsteps) ? 1 : 0;
     S *cap = (S *)a->capture;
+    if (traj_in) {
+      const wf::TrajBox b = wf::traj_box(a->traj_lo, a->traj_hi);
+      const int64_t slot = a->traj_slot0 + s + 1;
+      x.trE = (S *)a->traj_E + slot * 3 * b.nE;
+      x.trH = (S *)a->traj_H + slot * 3 * b.nH;
+    }
     hipLaunchKernelGGL(kern, dim3((unsigned)nb), dim3(threads), lds, st, g, m, Ebuf[cur],
                        Hbuf[cur], Ebuf[1 - cur], Hbuf[1 - cur], (S *)a->J, cf, dt, x, row, cap);
     WF_LAUNCH_CHECK();
-    if (a->traj_E) {
+    if (a->traj_E && !traj_in) {
       traj_store<S>(h, a, Ebuf[1 - cur], Hbuf[1 - cur], a->traj_slot0 + s + 1, st);
       WF_LAUNCH_CHECK();
     }

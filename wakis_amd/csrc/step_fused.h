@@ -33,6 +33,10 @@ struct FusedAux {
   // k_fused4: first tile along x, y, z of the launched tile range (ntx, nty,
   // ntz tiles from there); 0 for the whole grid
   int tx0, ty0, tz0;
+  // k_fused4 with escape codes, optional: the trajectory slots that this step
+  // fills (E on the cells [tlo, thi), H on [tlo - 1, thi))
+  void *trE, *trH;
+  int tlo[3], thi[3];
 };
 
 // z-face override of the face mask for components x and y at plane k:

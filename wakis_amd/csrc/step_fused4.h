@@ -540,6 +540,29 @@ __device__ __forceinline__ void fused4_tile(const GridDev &g, const MetricDev<S>
       stv_nt<V>(Eout, 2 * N + nk, En[2]);
       stv_nt<V>(Hout, nk, Hn[0]); stv_nt<V>(Hout, N + nk, Hn[1]);
       stv_nt<V>(Hout, 2 * N + nk, Hn[2]);
+      if constexpr (ESC) {
+        // the region's trajectory (a gather of its own took 3.3 us a step)
+        const bool kj = x.trE && k >= x.tlo[2] - 1 && k < x.thi[2] && j >= x.tlo[1] - 1 &&
+                        j < x.thi[1];
+        if (kj) {
+          const int ex = x.thi[0] - x.tlo[0], ey = x.thi[1] - x.tlo[1], ez = x.thi[2] - x.tlo[2];
+          const int64_t nE = (int64_t)ex * ey * ez;
+          const int64_t nH = (int64_t)(ex + 1) * (ey + 1) * (ez + 1);
+          const int jr = j - x.tlo[1], kr = k - x.tlo[2];
+#pragma unroll
+          for (int q = 0; q < V; ++q) {
+            const int ir = ic + q - x.tlo[0];
+            if (ir < -1 || ir >= ex) continue;
+            const int64_t rh = ir + 1 + (int64_t)(ex + 1) * (jr + 1 + (int64_t)(ey + 1) * (kr + 1));
+            const int64_t re = ir + (int64_t)ex * (jr + (int64_t)ey * kr);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+              ((S *)x.trH)[c * nH + rh] = Hn[c][q];
+              if (ir >= 0 && jr >= 0 && kr >= 0) ((S *)x.trE)[c * nE + re] = En[c][q];
+            }
+          }
+        }
+      }
       if (COND && !x.skip_j) {
         S Jn[3][V];
 #pragma unroll
