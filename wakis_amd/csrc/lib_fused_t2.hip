@@ -23,8 +23,8 @@ int fused_t2_applies(const wf_handle *h, const wf_step_args *a) {
     return 0;
   // Pairs are the faster launches at every size measured (us per step, one step
   // per launch against pairs: 32x32x64 FP32 16.0 / 7.5, 48x48x128 FP64 17.2 /
-  // 9.5, 91x75x161 FP32 35.0 / 17.6, 160x160x200 FP64 267 / 77, 300x220x180
-  // FP32 270 / 99). Where a call always ended with a single step, so that
+  // 8.6, 91x75x161 FP32 35.0 / 12.4, 160x160x200 FP64 267 / 58, 300x220x180
+  // FP32 270 / 66). Where a call always ended with a single step, so that
   // the spare buffers hold the fields one step back, it still does: rows that
   // are no whole number of lanes or longer than 256 cells, runs with a field
   // monitor and, by default (1), grids under 2^20 cells and FP64 rows under 224 cells.

@@ -50,17 +50,16 @@
 // each, no metric values, rings or scalars beside them; the row 0 of zeros stands
 // for cells off the grid.
 //
-// What bounds it: on material codes the instructions its 12 waves issue (664 of
-// 1,110 a plane are the arithmetic of the exact row sums, FP32); on weight codes
-// (408 of 663) the chain of loads, LDS passes and barriers of a plane beside the
-// memory. One branch per update and none per cell, buffer loads that return zeros
-// off the grid, own neighbours from registers. us per step, rows of one wave and
-// a branch per cell -> this form on material codes -> on weight codes:
-// 256x256x512 FP32 197 -> 188 -> 178 (1.70 GB per launch at 4.8 TB/s),
-// 200x200x400 FP32 with conduction 149 -> 111 -> 98, 256x256x128 FP64 134 ->
-// 106; and against one step per launch, which other rows took: 160x160x200 FP64
-// 267 -> 77, 300x220x180 FP32 270 -> 99 -> 90, 91x75x161 FP32 35 -> 17.6 -> 15.1,
-// 48x48x128 FP64 17.2 -> 9.4.
+// What bounds it: memory on large FP32 grids (256x256x512: 1.70 GB per launch at
+// 5.1 TB/s, the rate of a device copy); elsewhere the chain of a plane, LDS passes
+// and the instructions its 12 waves issue between two barriers (663 a plane on
+// weight codes, 408 of them the arithmetic of the exact row sums; 1,110 on material
+// codes). One branch per update and none per cell, buffer loads that return zeros
+// off the grid, own neighbours from registers. us per step, one step per launch (or
+// rows of one wave and a branch per cell, *) -> this form on material codes -> now:
+// 256x256x512 FP32 197* -> 188 -> 165, 200x200x400 FP32 with conduction 149* -> 111
+// -> 85, 300x220x180 FP32 270 -> 99 -> 66, 91x75x161 FP32 35 -> 17.6 -> 12.4,
+// 160x160x200 FP64 267 -> 66 -> 58, 48x48x128 FP64 17.2 -> 9.4 -> 8.6.
 #pragma once
 #include "step_fused4.h"
 #include "weight_codes.h"

@@ -596,6 +596,8 @@ class SolverFIT3D(RoutinesMixin):
         key = (self._lut_key, float(self.dt))
         if key == self._wkey:
             return self._wcode is not None
+        if torch.cuda.is_current_stream_capturing():
+            return False  # the table is made with a copy to the host: by a later call
         self._wkey, self._wcode, self._wtab = key, None, None
         n, nk = _lib.WF_WEIGHT_ROW, 27 * self._nmat
         buf = torch.empty(nk * n + nk + 1, dtype=torch.int32, device=self.device)
