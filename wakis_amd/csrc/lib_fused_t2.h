@@ -144,6 +144,13 @@ inline bool t2_weights(const wf_handle *h, const wf_step_args *a) {
 }
 
 inline void t2_aux(const T2Shape &sh, const wf::GridDev &g, const wf_step_args *a, wf::T2Aux &x) {
+  // FP32 stores streamed past the caches where tiles write whole 128-byte lines and
+  // E and H with their spare buffers about fill the 256 MB of last-level cache. ms a
+  // pass, streamed against not: 256x256x512 597 / 620, 160x160x200 39.5 / 40.2, but
+  // 128x128x160 21.1 / 18.7, 96x96x160 with a monitor 24.7 / 23.6, and on part lines
+  // 300x220x180 71.6 / 67.1, 200x200x400 with conduction 153.6 / 151.2. FP64 always:
+  // 160x160x200 82.2 / 84.3, 48x48x128 19.7 / 20.9.
+  x.stream = g.Nx % 32 == 0 && (sh.ntx == 1 || sh.OW % 32 == 0) && 48.0 * (double)g.N > 200e6;
   x.ixs = a->ixs;
   x.iys = a->iys;
   x.cap_ix0 = a->cap_ix0; x.cap_iy0 = a->cap_iy0; x.cap_nx = a->cap_nx; x.cap_ny = a->cap_ny;

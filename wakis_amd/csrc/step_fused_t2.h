@@ -75,6 +75,7 @@ struct T2Aux {
   int T, OW;              // own rows and cells of a tile
   int Q, QS;              // lanes and LDS slots of a staged row
   int l0, ln;             // own lanes of a row: l0 .. l0 + ln - 1, lane l0 at the tile's first cell
+  int stream;             // FP32: stores are streamed past the caches
   int skip_j;             // COND: 1 = J is stored by a later launch of the call
 };
 
@@ -132,14 +133,10 @@ __device__ __forceinline__ void buf_ld(Buf b, const Offs<V> &o, bool in, uint32_
       for (int q = 0; q < V - 1; ++q) d[c][q] = buf_ld1<S>(b, o.c[q], s + c * cstep);
   }
 }
-// the same for stores: FP64 streamed past the caches (cache policy 2:
-// non-temporal), FP32 not. ms a pass, streamed against not: 300x220x180 FP32 71.6 /
-// 67.1, 200x200x400 FP32 with conduction 153.6 / 151.2, 96x96x160 FP32 with a
-// monitor 24.4 / 23.6; 160x160x200 FP64 82.2 / 84.3, 48x48x128 FP64 19.7 / 20.9
-template <bool RAG, typename S, int NC, int V>
-__device__ __forceinline__ void buf_st(Buf b, const Offs<V> &o, uint32_t s, uint32_t cstep,
-                                       const S (&d)[NC][V]) {
-  constexpr int POL = sizeof(S) == 8 ? 2 : 0;
+// the same for stores, with cache policy POL (2: non-temporal)
+template <int POL, bool RAG, typename S, int NC, int V>
+__device__ __forceinline__ void buf_st_pol(Buf b, const Offs<V> &o, uint32_t s, uint32_t cstep,
+                                           const S (&d)[NC][V]) {
   typedef S vec __attribute__((ext_vector_type(V)));
   typedef unsigned int u4 __attribute__((ext_vector_type(4)));
 #pragma unroll
@@ -165,6 +162,14 @@ __device__ __forceinline__ void buf_st(Buf b, const Offs<V> &o, uint32_t s, uint
               b, (int)o.c[q], (int)(s + c * cstep), POL);
       }
   }
+}
+
+// FP64 is always streamed past the caches, FP32 on the host's rule (t2_aux)
+template <bool RAG, typename S, int NC, int V>
+__device__ __forceinline__ void buf_st(bool stream, Buf b, const Offs<V> &o, uint32_t s,
+                                       uint32_t cstep, const S (&d)[NC][V]) {
+  if (sizeof(S) == 8 || stream) buf_st_pol<2, RAG>(b, o, s, cstep, d);
+  else buf_st_pol<0, RAG>(b, o, s, cstep, d);
 }
 
 // Dynamic LDS of a workgroup in values of S: the ring of iAy / itAy rows, the
@@ -554,7 +559,7 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
       if (capq0 < capq1 && x.cap_sample < x.cap_samples && k >= k0 && k < kend)
         capture(k, E1[2]);
       if (MON && k >= k0 && k < kend)  // E of the first step, for a field monitor
-        buf_st<RAG>(buf_of(E1out, 3 * NB), ofs, (I)k * sz * ES, NB, E1);
+        buf_st<RAG>(x.stream != 0, buf_of(E1out, 3 * NB), ofs, (I)k * sz * ES, NB, E1);
     }
     if (doH2 && p >= kstart) {  // H2 below plane 0 stays 0
       const Metric o = metric(0, rp, p);
@@ -578,7 +583,7 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
         if (q == V - 1) h2(1, Pd, q) = H2[1][q];
       }
       // H2(k-1) of the own rows is final
-      if (l2e) buf_st<RAG>(bHo, ofs, (I)p * sz * ES, NB, H2);
+      if (l2e) buf_st<RAG>(x.stream != 0, bHo, ofs, (I)p * sz * ES, NB, H2);
     }
 #pragma unroll
     for (int c = 0; c < 3; ++c)
@@ -640,7 +645,7 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
         if (!COND) J[2 * g.N + (int64_t)p * g.sz + cell + qbeam] = bv2;
       }
       if (capq0 < capq1 && x.cap_sample + 1 < x.cap_samples) capture(g.Nz + p, E2[2]);
-      buf_st<RAG>(bEo, ofs, (I)p * sz * ES, NB, E2);
+      buf_st<RAG>(x.stream != 0, bEo, ofs, (I)p * sz * ES, NB, E2);
       if (COND && !x.skip_j) {  // J = sigma E2 by the call's last launch
         const Buf bJ = buf_of(J, 3 * NB);
 #pragma unroll
@@ -649,7 +654,7 @@ t2_tile(const GridDev &g, const MetricDev<S> &m, const S *__restrict__ Ein,
 #pragma unroll
           for (int c = 0; c < 3; ++c) Jn[c][q] = (S)(t[SG + c] * E2[c][q]);
         }
-        buf_st<RAG>(bJ, ofs, (I)p * sz * ES, NB, Jn);
+        buf_st<RAG>(x.stream != 0, bJ, ofs, (I)p * sz * ES, NB, Jn);
       }
     }
 #pragma unroll
