@@ -18,7 +18,7 @@ using Fused4Fn = void (*)(wf::GridDev, wf::MetricDev<S>, const S *, const S *, S
 
 // k_fused4, or k_fused4_wide (64-bit offsets) for arrays past 4 GiB
 template <typename S, int JM, bool CO, bool LU, bool DE, int TY, bool MK, int V, bool FR,
-          bool ES, bool WIDE>
+          int ES, bool WIDE>
 Fused4Fn<S> fused4_ptr() {
   if constexpr (WIDE) return &wf::k_fused4_wide<S, JM, CO, LU, DE, TY, MK, V>;
   else return &wf::k_fused4<S, JM, CO, LU, DE, TY, MK, V, FR, ES>;
@@ -27,7 +27,7 @@ Fused4Fn<S> fused4_ptr() {
 // The k_fused4 instantiation for the step's J mode, conductivity, coefficient
 // form, boundary order and masking.
 template <typename S, int TY, int V, bool FR, bool WIDE = false>
-Fused4Fn<S> pick_fused4(bool lut, bool cond, bool jline, bool desc, bool mk, bool esc = false) {
+Fused4Fn<S> pick_fused4(bool lut, bool cond, bool jline, bool desc, bool mk, int esc = 0) {
 #define WF_PICK(JM, CO, LU, ES)                                                             \
   do {                                                                                      \
     if (desc) return mk ? fused4_ptr<S, JM, CO, LU, true, TY, true, V, FR, ES, WIDE>()      \
@@ -36,21 +36,46 @@ Fused4Fn<S> pick_fused4(bool lut, bool cond, bool jline, bool desc, bool mk, boo
               : fused4_ptr<S, JM, CO, LU, false, TY, !LU, V, FR, ES, WIDE>();               \
   } while (0)
   if constexpr (!WIDE) {
+    if constexpr (!FR) {
+      if (esc == 2) {  // a run with the trajectory in the step (traj_in_step)
+        if (cond)
+          return desc ? fused4_ptr<S, 0, true, true, true, TY, false, V, FR, 2, WIDE>()
+                      : fused4_ptr<S, 0, true, true, false, TY, false, V, FR, 2, WIDE>();
+        return desc ? fused4_ptr<S, 1, false, true, true, TY, false, V, FR, 2, WIDE>()
+                    : fused4_ptr<S, 1, false, true, false, TY, false, V, FR, 2, WIDE>();
+      }
+    }
     if (lut && esc) {
-      if (cond) WF_PICK(0, true, true, true);
-      if (jline) WF_PICK(1, false, true, true);
-      WF_PICK(0, false, true, true);
+      if (cond) WF_PICK(0, true, true, 1);
+      if (jline) WF_PICK(1, false, true, 1);
+      WF_PICK(0, false, true, 1);
     }
   }
   if (lut) {
-    if (cond) WF_PICK(0, true, true, false);
-    if (jline) WF_PICK(1, false, true, false);
-    WF_PICK(0, false, true, false);
+    if (cond) WF_PICK(0, true, true, 0);
+    if (jline) WF_PICK(1, false, true, 0);
+    WF_PICK(0, false, true, 0);
   }
-  if (cond) WF_PICK(0, true, false, false);
-  if (jline) WF_PICK(1, false, false, false);
-  WF_PICK(0, false, false, false);
+  if (cond) WF_PICK(0, true, false, 0);
+  if (jline) WF_PICK(1, false, false, 0);
+  WF_PICK(0, false, false, 0);
 #undef WF_PICK
+}
+
+// Whether the step kernel itself fills the trajectory slots of a run on escape
+// codes (ESC 2), rather than a gather after it. The gather is a launch of 2 to 3
+// us; in the step, the few workgroups that own the block store its cells one at a
+// time on their march. Up to 2^19 cells the launch is the larger part (us a step, in
+// the step / gathered: 40x40x64 FP32 9.2 / 10.9, 64x64x96 FP32 12.0 / 13.6, FP64
+// 17.4 / 19.5). Above, the march is: 72x72x112 FP32 28.2 / 26.9, 128x128x256 99.5 /
+// 95.3. The extra registers cost more still where fewer workgroups then fit a CU
+// (72x72x112 FP64 with conduction 57 / 37, 128x128x256 205 / 138): gathered. The
+// launched tiles of a box have to hold the whole block and the plane below it.
+inline bool traj_in_step(const wf_handle *h, const wf_step_args *a, bool lut, bool box) {
+  for (int d = 0; box && d < 3; ++d)
+    if (a->box_lo[d] > a->traj_lo[d] - 1 || a->box_hi[d] < a->traj_hi[d]) return false;
+  return a->traj_E && lut && a->code_escape && a->zero_masked &&
+         (a->conductive || a->jmode == WF_J_LINE) && h->g.N <= (int64_t)1 << 19;
 }
 
 template <typename S, int TY, int V, bool FR, bool WIDE>
@@ -84,13 +109,21 @@ int step_fused4(wf_handle *h, wf_step_args *a, const wf::MetricDev<S> &m, hipStr
     x.ntx = (g.Nx + Wc - 1) / Wc;
     x.nty = (g.Ny + TY - 1) / TY;
   }
-  const Fused4Fn<S> kern = pick_fused4<S, TY, V, FR, WIDE>(lut, a->conductive != 0,
-                                                      a->jmode == WF_J_LINE, g.m1desc != 0,
-                                                      !(lut && a->zero_masked),
-                                                      lut && a->code_escape);
   // optional box: launch only the tiles that meet it
   const bool box = a->box_hi[0] > a->box_lo[0] && a->box_hi[1] > a->box_lo[1] &&
                    a->box_hi[2] > a->box_lo[2];
+  const auto pick = [&](int esc) {
+    return pick_fused4<S, TY, V, FR, WIDE>(lut, a->conductive != 0, a->jmode == WF_J_LINE,
+                                           g.m1desc != 0, !(lut && a->zero_masked), esc);
+  };
+  Fused4Fn<S> kern = pick(lut && a->code_escape ? 1 : 0);
+  bool traj_in = false;
+  if (!FR && !WIDE && traj_in_step(h, a, lut, box)) {
+    const Fused4Fn<S> k2 = pick(2);
+    traj_in = fused_occupancy(h, (const void *)k2, threads, lds) >=
+              fused_occupancy(h, (const void *)kern, threads, lds);
+    if (traj_in) kern = k2;
+  }
   x.tx0 = x.ty0 = x.tz0 = 0;
   if (box) {
     const int W = FR ? g.Nx : 64 * V, R = FR ? fr_rows : TY;
@@ -136,8 +169,6 @@ int step_fused4(wf_handle *h, wf_step_args *a, const wf::MetricDev<S> &m, hipStr
     cf.iAx = t; cf.iAy = t + yz; cf.iAz = t + yz + xz;
     cf.itAx = t + yz + xz + xy; cf.itAy = cf.itAx + yz; cf.itAz = cf.itAy + xz;
   }
-  // escape kernels fill the trajectory themselves
-  const bool traj_in = !WIDE && lut && a->code_escape && a->traj_E;
   for (int d = 0; d < 3; ++d) { x.tlo[d] = a->traj_lo[d]; x.thi[d] = a->traj_hi[d]; }
   int cur = 0;
   for (int s = 0; s < a->nsteps; ++s) {

@@ -33,7 +33,7 @@ struct FusedAux {
   // k_fused4: first tile along x, y, z of the launched tile range (ntx, nty,
   // ntz tiles from there); 0 for the whole grid
   int tx0, ty0, tz0;
-  // k_fused4 with escape codes, optional: the trajectory slots that this step
+  // k_fused4 with escape codes (ESC 2): the trajectory slots that this step
   // fills (E on the cells [tlo, thi), H on [tlo - 1, thi))
   void *trE, *trH;
   int tlo[3], thi[3];

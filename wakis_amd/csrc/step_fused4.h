@@ -121,7 +121,7 @@ __device__ __forceinline__ int xcd_tile(int blin, int nb) {
 // WIDE: 64-bit element offsets (arrays past 4 GiB); otherwise 32-bit byte
 // offsets from the array base (every 3N array within 4 GiB).
 template <typename S, int JM, bool COND, bool LUT, bool DESC, int TY, bool MK, int V, bool FR,
-          bool ESC, bool WIDE = false>
+          int ESC, bool WIDE = false>
 __device__ __forceinline__ void fused4_tile(const GridDev &g, const MetricDev<S> &m,
                                             const S *__restrict__ Ein, const S *__restrict__ Hin,
                                             S *__restrict__ Eout, S *__restrict__ Hout,
@@ -540,9 +540,8 @@ __device__ __forceinline__ void fused4_tile(const GridDev &g, const MetricDev<S>
       stv_nt<V>(Eout, 2 * N + nk, En[2]);
       stv_nt<V>(Hout, nk, Hn[0]); stv_nt<V>(Hout, N + nk, Hn[1]);
       stv_nt<V>(Hout, 2 * N + nk, Hn[2]);
-      if constexpr (ESC) {
-        // the region's trajectory (a gather of its own took 3.3 us a step)
-        const bool kj = x.trE && k >= x.tlo[2] - 1 && k < x.thi[2] && j >= x.tlo[1] - 1 &&
+      if constexpr (ESC == 2) {  // the region's trajectory
+        const bool kj = k >= x.tlo[2] - 1 && k < x.thi[2] && j >= x.tlo[1] - 1 &&
                         j < x.thi[1];
         if (kj) {
           const int ex = x.thi[0] - x.tlo[0], ey = x.thi[1] - x.tlo[1], ez = x.thi[2] - x.tlo[2];
@@ -594,9 +593,10 @@ __device__ __forceinline__ void fused4_tile(const GridDev &g, const MetricDev<S>
 // FR: TY only bounds the workgroup (64 * (TY + 1) threads); x.rows is the tile
 // ESC (with LUT): material code 255 marks cells whose coefficients are read
 // from the arrays a, b, ieps, sigma (per-cell parameters, e.g. a block of
-// cells being optimised); the table then has at most 255 rows
+// cells being optimised); the table then has at most 255 rows. ESC 2: the step
+// also fills the region's trajectory slots (x.trE, x.trH; traj_in_step says when)
 template <typename S, int JM, bool COND, bool LUT, bool DESC, int TY, bool MK, int V, bool FR,
-          bool ESC = false>
+          int ESC = 0>
 __global__ void __launch_bounds__(64 * (TY + 1))
 k_fused4(GridDev g, MetricDev<S> m, const S *__restrict__ Ein, const S *__restrict__ Hin,
          S *__restrict__ Eout, S *__restrict__ Hout, S *__restrict__ J, Coefs<S> cf, S dt,
@@ -614,7 +614,7 @@ k_fused4_wide(GridDev g, MetricDev<S> m, const S *__restrict__ Ein, const S *__r
               S *__restrict__ Eout, S *__restrict__ Hout, S *__restrict__ J, Coefs<S> cf, S dt,
               FusedAux x, const S *__restrict__ beam_row, S *__restrict__ cap) {
   const int tile = xcd_tile(blockIdx.x, x.ntx * x.nty * x.ntz);
-  fused4_tile<S, JM, COND, LUT, DESC, TY, MK, V, false, false, true>(
+  fused4_tile<S, JM, COND, LUT, DESC, TY, MK, V, false, 0, true>(
       g, m, Ein, Hin, Eout, Hout, J, cf, dt, x, beam_row, cap, tile);
 }
 
@@ -677,7 +677,7 @@ k_fused4_batch(const BatchDesc<S> *__restrict__ d, int ninst, int ntiles,
   x.cap_sample = b.cap_sample0 + step;
   x.skip_j = (step + 1 < b.nsteps) ? 1 : 0;
   const S *row = b.beam_table ? b.beam_table + (b.beam_row0 + step) * b.g.Nz : nullptr;
-  fused4_tile<S, JM, COND, LUT, DESC, TY, MK, V, FR, false>(
+  fused4_tile<S, JM, COND, LUT, DESC, TY, MK, V, FR, 0>(
       b.g, b.m, odd ? b.E2 : b.E, odd ? b.H2 : b.H, odd ? b.E : b.E2, odd ? b.H : b.H2, b.J,
       b.cf, b.dt, x, row, b.cap, tile - b.tile0);
 }
