@@ -291,15 +291,18 @@ int fused_occupancy(wf_handle *h, const void *kern, int threads, size_t lds) {
 // workgroup marches KZ + 1 planes, each a chain of loads and two barriers: one
 // workgroup on a CU takes the chain's time per plane, r of them the longer of it
 // and r times the share of it that their waves need (0.05 a wave and 0.0065 per
-// byte of a lane's row, at most 0.95: from 0.4 for 4 waves of one double on).
+// byte of a lane's row, at most 0.95: from 0.4 for 4 waves of one double on). Where
+// a CU holds only one, they run in turn: 0.95 (FP32 rows of two cells a lane, escape
+// codes with conduction, 5 planes in two rounds against 9 in one: 96x96x160 45.2 /
+// 43.0 us, 110x110x140 46.8 / 44.9).
 // Within 4% of the best of KZ = 1 .. 64 on 20 grids of one step per launch and 6
 // of the reverse step (9% on one). The former rule, at least 8 planes per
 // workgroup, took 15.9 us per step against 7.9 at 40x40x64 FP32, 17.4 / 13.1 at
 // 48x48x128 FP64, 213 / 152 at 160x160x160 FP64, and 17.3 ms against 10.9 for the
 // 720 FP32 reverse steps at 64x64x96; from 256x256x256 on both are within 3%.
 int auto_kz(int64_t nxy, int Nz, int64_t conc, int ncu, int waves, int lane_bytes) {
-  const double share = std::min(0.95, waves * (0.05 + 0.0065 * lane_bytes));
   const double per_cu = std::max<double>(1.0, (double)(conc / ncu));
+  const double share = per_cu < 2 ? 0.95 : std::min(0.95, waves * (0.05 + 0.0065 * lane_bytes));
   double best = 1e300;
   int kz = 1;
   for (int k = 1; k <= std::min(Nz, 64); ++k) {
