@@ -23,7 +23,7 @@ SOURCES = ["lib_fused_f32_a.hip", "lib_fused_f32_b.hip", "lib_fused_f32_c.hip",
            "lib_batch.hip", "lib_batch_t2.hip", "lib_adjoint.hip", "lib_core.hip"]
 HEADERS = ["lib_internal.h", "lib_fused.h", "lib_fused_t2.h", "fit_common.h",
            "step_general.h", "step_fused.h",
-           "step_fused4.h", "step_fused_t2.h", "wake.h", "reduce.h", "adjoint.h",
+           "step_fused4.h", "step_fused_t2.h", "t2_limits.h", "wake.h", "reduce.h", "adjoint.h",
            "adjoint_fused.h", "monitor.h", "weight_codes.h"]
 
 # -ffp-contract=off keeps every multiply and add separately rounded, as numpy

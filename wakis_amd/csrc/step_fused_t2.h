@@ -62,6 +62,7 @@
 // 160x160x200 FP64 267 -> 66 -> 58, 48x48x128 FP64 17.2 -> 9.4 -> 8.6.
 #pragma once
 #include "step_fused4.h"
+#include "t2_limits.h"
 #include "weight_codes.h"
 
 namespace wf {
@@ -89,8 +90,7 @@ struct T2Slots {
 // An array behind a buffer descriptor: a lane addresses it with a byte offset
 // of its own plus a uniform one (plane and component), so a plane's accesses
 // need no address arithmetic, and a lane whose own offset is OOB reads zeros
-// and writes nothing, so they need no branch.
-constexpr uint32_t OOB = 0xfffffff0u;
+// and writes nothing, so they need no branch (t2_limits.h).
 typedef __amdgpu_buffer_rsrc_t Buf;
 __device__ __forceinline__ Buf buf_of(const void *p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, (int)bytes, 0x00020000);

@@ -863,9 +863,14 @@ class SolverFIT3D(RoutinesMixin):
         size = np.dtype(self.dtype).itemsize
         box = all(h > l for l, h in zip(args.box_lo, args.box_hi))
         return bool(args.two_step and args.code and args.zero_masked and not args.code_escape
-                    and args.beam_table and 3 * self.N * size < 2 ** 32 and args.variant == 0
+                    and args.beam_table and self._pairs_in_reach() and args.variant == 0
                     and args.full_rows <= 0 and args.cells_per_lane in (0, 16 // size)
                     and not box and not args.traj_E and (not args.mon_acc or args.mon_work))
+
+    def _pairs_in_reach(self):
+        """Whether the two-step kernel's 32-bit offsets reach every array (t2_limits.h)."""
+        tables = 2 * (self.Ny * self.Nz + self.Nx * self.Nz + self.Nx * self.Ny)
+        return max(3 * self.N, tables) * np.dtype(self.dtype).itemsize <= 0xfffffff0
 
     def _monitor_work(self):
         """Scratch for the E of up to eight steps of a monitored run (7, 3 or 1
