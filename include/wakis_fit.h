@@ -183,8 +183,8 @@ typedef struct wf_step_args {
    * material codes with zero_masked and no escape code, the beam line fed
    * from beam_table (with or without conduction), row segments (variant 0,
    * full_rows <= 0, cells_per_lane 0 or 16 bytes of cells), every 3N array
-   * and the metric2d tables at most 2^32 - 16 bytes, no box, no trajectory, no monitor without mon_work; otherwise one step per
-   * launch. Results are identical to one step per launch. 0 = one step per
+   * at most 2^32 - 16 bytes, no box, no trajectory, no monitor without mon_work;
+   * otherwise one step per launch. Results are identical to one step per launch. 0 = one step per
    * launch; 4 or 8: two steps per launch with at most that many rows per
    * workgroup.
    * E2 and H2 hold the fields one step back after a call, except (fields two

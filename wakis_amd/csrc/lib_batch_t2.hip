@@ -22,7 +22,7 @@ int build(const wf::BatchDesc<S> *bd, wf_handle *const *hs, const wf_step_args *
     const wff::T2Shape sh = wff::t2_shape<S>(g, t->wc ? as[i].nw : as[i].nmat, t->wc != 0,
                                              std::min(share, ncu), 0, 0,
                                              std::max(0, ncu - share));
-    if (!sh.ok || !wf::t2_in_reach(g.Nx, g.Ny, g.Nz, sizeof(S))) return 0;
+    if (!sh.ok || !wf::t2_in_reach(g.N, sizeof(S))) return 0;
     d[i].b = bd[i];
     if (t->wc) {
       wf::Coefs<S> &cf = d[i].b.cf;

@@ -17,7 +17,7 @@ int fused_t2_applies(const wf_handle *h, const wf_step_args *a) {
                                                    : a->jmode == WF_J_LINE);
   const int elem = h->dtype == WF_F64 ? 8 : 4, vn = 16 / elem;  // cells per lane
   if (a->two_step == 0 || !lut || !a->zero_masked || a->code_escape || a->compute_f64 || !jok ||
-      !wf::t2_in_reach(g.Nx, g.Ny, g.Nz, elem) || a->variant != 0 ||
+      !wf::t2_in_reach(g.N, elem) || a->variant != 0 ||
       a->full_rows > 0 || (a->cells_per_lane != 0 && a->cells_per_lane != vn) || box ||
       a->traj_E || (a->mon_acc && (!a->mon_work || a->mon_slots < 1)) || a->nsteps < 2)
     return 0;

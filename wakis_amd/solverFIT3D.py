@@ -869,8 +869,7 @@ class SolverFIT3D(RoutinesMixin):
 
     def _pairs_in_reach(self):
         """Whether the two-step kernel's 32-bit offsets reach every array (t2_limits.h)."""
-        tables = 2 * (self.Ny * self.Nz + self.Nx * self.Nz + self.Nx * self.Ny)
-        return max(3 * self.N, tables) * np.dtype(self.dtype).itemsize <= 0xfffffff0
+        return 3 * self.N * np.dtype(self.dtype).itemsize <= 0xfffffff0
 
     def _monitor_work(self):
         """Scratch for the E of up to eight steps of a monitored run (7, 3 or 1
