@@ -592,13 +592,25 @@ class SolverFIT3D(RoutinesMixin):
         """Weight codes for the two-step kernel (wf_step_args.wcode): per cell a
         row of the products of metric, material and dt, where the metric is
         uniform along each axis but for its first and last cells and at most 255
-        distinct rows occur. Valid as long as the material codes and dt."""
+        distinct rows occur. Valid as long as the material codes and dt. Without
+        memory for them the run does without, on material codes."""
         key = (self._lut_key, float(self.dt))
         if key == self._wkey:
             return self._wcode is not None
         if torch.cuda.is_current_stream_capturing():
             return False  # the table is made with a copy to the host: by a later call
-        self._wkey, self._wcode, self._wtab = key, None, None
+        self._wkey = self._wcode = self._wtab = None
+        try:
+            made = self._make_weight_table()
+        except torch.OutOfMemoryError:
+            made = None
+        if made is not None:
+            self._wcode, self._wtab = made
+        self._wkey = key
+        return made is not None
+
+    def _make_weight_table(self):
+        """(codes, table) for the present materials and dt, or None."""
         n, nk = _lib.WF_WEIGHT_ROW, 27 * self._nmat
         buf = torch.empty(nk * n + nk + 1, dtype=torch.int32, device=self.device)
         lib, st = _lib.lib(), _lib.stream_ptr()
@@ -609,22 +621,22 @@ class SolverFIT3D(RoutinesMixin):
         host = buf.cpu().numpy()
         rows, used = host[:nk * n].reshape(nk, n), host[nk * n:]
         if used[nk]:
-            return False
+            return None
         sel = np.flatnonzero(used[:nk])
         distinct, inv = np.unique(rows[sel], axis=0, return_inverse=True)
         if len(distinct) > 255:
-            return False
+            return None
         table = np.zeros((len(distinct) + 1, n), dtype=np.int32)  # row 0: cells off the grid
         table[1:] = distinct
         row_of = np.zeros(nk, dtype=np.uint8)
         row_of[sel] = 1 + inv.reshape(-1)
         row_of = torch.as_tensor(row_of, device=self.device)
-        self._wcode = torch.empty(self.N, dtype=torch.uint8, device=self.device)
-        self._wtab = torch.as_tensor(table.view(np.float32), device=self.device)
+        wcode = torch.empty(self.N, dtype=torch.uint8, device=self.device)
+        wtab = torch.as_tensor(table.view(np.float32), device=self.device)
         _lib.check(lib.wf_weight_codes(self._handle, _lib.ptr(self._code), self._nmat,
-                                       _lib.ptr(row_of), _lib.ptr(self._wcode), st),
+                                       _lib.ptr(row_of), _lib.ptr(wcode), st),
                    "wf_weight_codes")
-        return True
+        return wcode, wtab
 
     def _masked_zero(self):
         """True if E is zero on every PEC-masked edge, H on every PMC-masked
