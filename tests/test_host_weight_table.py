@@ -111,3 +111,44 @@ def test_run_goes_on_without_memory_for_the_table(kernels, monkeypatch):
     assert a.code and not a.wcode and a.nw == 0
     n = len(kernels.calls)
     assert s._prepare_fused(_args(s)) and len(kernels.calls) == n  # not tried again
+
+
+def _no_pairs():
+    """Calls that run one step per launch."""
+    yield "trajectory", dict(traj_E=8)
+    yield "box", dict(box_hi=(3, 3, 3))
+    yield "monitor without scratch", dict(mon_acc=8)
+    yield "no beam table", dict(beam_table=None)
+    for name, v in (("fused_variant", 1), ("fused_full_rows", 2), ("fused_cells_per_lane", 1),
+                    ("fused_two_step", 0), ("skip_masks", False)):
+        yield name, {name: v}
+
+
+def test_no_table_for_calls_of_single_steps(kernels):
+    s = _solver()
+    for name, kw in _no_pairs():
+        a, held = _args(s), {}
+        for k, v in kw.items():
+            if hasattr(s, k):
+                held[k] = getattr(s, k)
+                setattr(s, k, v)
+            elif isinstance(v, tuple):
+                getattr(a, k)[:] = v
+            else:
+                setattr(a, k, v)
+        assert s._prepare_fused(a) and a.code and not a.wcode, name
+        for k, v in held.items():
+            setattr(s, k, v)
+    assert kernels.calls == []
+    short = _args(s, 40)
+    assert s._prepare_fused(short) and not short.wcode and kernels.calls == []
+    a = _args(s)
+    assert s._prepare_fused(a) and a.wcode and kernels.calls == ["rows", "codes"]
+    short = _args(s, 40)  # made already
+    assert s._prepare_fused(short) and short.wcode and kernels.calls == ["rows", "codes"]
+    s.ieps[2:5, 2:5, 2:5, "x"] = 1e10  # new materials: again by the first longer call
+    s.update_tensors()
+    short = _args(s, 40)
+    assert s._prepare_fused(short) and not short.wcode and kernels.calls == ["rows", "codes"]
+    a = _args(s)
+    assert s._prepare_fused(a) and a.wcode and len(kernels.calls) == 4

@@ -791,9 +791,9 @@ class SolverFIT3D(RoutinesMixin):
             args.code_escape = int(self._code_escape)
             # weight codes where pairs of steps run: built by the first longer call
             # (100 to 200 us, a few steps' gain at any size), then kept
-            if (self.use_weight_codes and args.two_step and args.beam_table and args.zero_masked
-                    and self.dtype == np.float32 and not self._code_escape
-                    and (args.nsteps >= 64 or self._wkey is not None)
+            if (self.use_weight_codes and self.dtype == np.float32
+                    and self._pairs_apply(args, prepared=True)
+                    and (args.nsteps >= 64 or self._wkey == (self._lut_key, float(self.dt)))
                     and self._weight_table()):
                 args.wcode, args.wtab = _lib.ptr(self._wcode), _lib.ptr(self._wtab)
                 args.nw = self._wtab.shape[0]
