@@ -195,10 +195,10 @@ typedef struct wf_step_args {
   int32_t two_step;
   int32_t two_step_used;  /* out: two steps per launch, 1: to the call's end (but an
                            * odd step), 2: up to its single last steps            */
-  /* Optional with mon_acc: device scratch of mon_slots (1, 3 or 7) times 3N
+  /* Optional with mon_acc: device scratch of mon_slots (1, 3, 5 or 7) times 3N
    * values of the storage type. Where the two-step kernel applies, the
-   * accumulators then cross memory once per 2, 4 or 8 steps; same results, the
-   * call's last step or two singly. */
+   * accumulators then cross memory once per mon_slots + 1 steps; same results,
+   * the call's last step or two singly. */
   void *mon_work;
   int32_t mon_slots;
   /* Optional with code, FP32 storage, two steps per launch: per cell a weight

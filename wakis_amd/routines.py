@@ -166,14 +166,16 @@ class RoutinesMixin:
                                  "and a checkpoint file name")
         ctx = self._wake_setup(wakelength, compute_plane)
         Nt = ctx["Nt"]
-        if Nt >= 2000 and self.N >= (1 << 22):
+        per_call = min(1 if callback is not None else Nt if chunk is None else int(chunk),
+                       Nt if every is None else every)
+
+        def pairs():
+            return per_call >= 3 and self._pairs_apply(self._wake_args(ctx, 0, 3))
+        if Nt >= 2000 and self.N >= (1 << 22) and not pairs():
             # long run: measure the kernel shapes first, unless it takes two steps
             # per launch, which no shape of one step per launch beats (the trials
             # took 44 of 712 ms of a 3,600-step run at 256x256x512)
-            per_call = min(1 if callback is not None else Nt if chunk is None else int(chunk),
-                           Nt if every is None else every)
-            if per_call < 3 or not self._pairs_apply(self._wake_args(ctx, 0, 3)):
-                self.tune_fused(lambda k: self._wake_args(ctx, 0, k))
+            self.tune_fused(lambda k: self._wake_args(ctx, 0, k))
         if save_J:  # J_z on the window before the run, for Jz.h5
             ix0, iy0, nx, ny = ctx["win"]
             ctx["J0"] = self.J.to_matrix("z")[ix0:ix0 + nx, iy0:iy0 + ny, :].reshape(
@@ -182,7 +184,8 @@ class RoutinesMixin:
         print("Running electromagnetic time-domain simulation...")
         t0 = time.time()
         monitor = field_monitor if (use_field_monitor and field_monitor is not None) else None
-        work = self._monitor_work() if monitor is not None else None
+        self._monitor_pairs = (per_call - 1) // 2  # of a call: its last step is single
+        work = self._monitor_work() if monitor is not None and pairs() else None
         per_step = callback is not None
         step = 1 if per_step else (Nt if chunk is None else int(chunk))
         while n < Nt:

@@ -216,6 +216,7 @@ class SolverFIT3D(RoutinesMixin):
         self._wlive_key = None
         self.use_weight_codes = True
         self._wkey = self._wcode = self._wtab = None
+        self._monitor_pairs = 4
         self._code = self._mat = self._metric2d = None
         self._nmat = 0
         self.update_tensors("all", _initial=True)
@@ -885,12 +886,13 @@ class SolverFIT3D(RoutinesMixin):
 
     def _monitor_work(self):
         """Scratch for the E of up to eight steps of a monitored run (7, 3 or 1
-        arrays of 3N values, at most a quarter of the free device memory), or
-        None."""
+        arrays of 3N values, or as many as ``_monitor_pairs`` pairs of steps
+        need; at most a quarter of the free device memory), or None."""
         free, _ = torch.cuda.mem_get_info(self.device)
         one = self.E.array.numel() * self.E.array.element_size()
-        for slots in (7, 3, 1):
-            if slots * one <= free // 4:
+        need = 2 * min(self._monitor_pairs, 4) - 1
+        for slots in (need, 3, 1):
+            if slots <= need and slots * one <= free // 4:
                 return torch.empty((slots, self.E.array.numel()), dtype=self.E.array.dtype,
                                    device=self.device)
         return None
