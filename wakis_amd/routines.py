@@ -121,6 +121,8 @@ class RoutinesMixin:
             k = min(size, Nt - 1 - n)
             val = np.array([[float(v) for v in source._values(i * self.dt)]
                             for i in range(n, n + k)]).T.copy()
+            if np.any(np.isfinite(val) & (np.abs(val) > np.finfo(self.dtype).max)):
+                return n  # Field refuses a value past the storage type
             self.E.version += k
             self.H.version += k
             args = self._step_args(k)
