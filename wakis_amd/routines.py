@@ -97,9 +97,12 @@ class RoutinesMixin:
         steps taken (0: none). For runs whose every step takes the exact general
         path: a conductive grid (a write to E ends J = sigma E) or one whose
         flat-index wrap terms couple live cells whatever the fields hold."""
+        from .solverFIT3D import SolverFIT3D
         from .sources import PlaneWave
         if type(source) is not PlaneWave or "update" in vars(source):
             return 0
+        if getattr(self.one_step, "__func__", None) is not SolverFIT3D.one_step:
+            return 0  # the caller's own step
         if self.path == "fused" or self.keep_previous_fields or not (
                 self.path == "general" or self.use_conductivity
                 or self._jmode() == _lib.WF_J_FULL or self._compute_f64()
