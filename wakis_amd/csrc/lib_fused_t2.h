@@ -171,8 +171,11 @@ int launch_t2(wf_handle *h, wf_step_args *a, const wf::MetricDev<S> &m, hipStrea
   const T2Shape sh =
       t2_shape<S>(g, nrows, wc, h->ncu, a->two_step > 1 ? a->two_step : 0, a->kz);
   if (!sh.ok) {  // one step per launch
-    a->two_step = 0;
-    return sizeof(S) == 4 ? step_fused_f32(h, a, st) : step_fused_f64(h, a, st);
+    wf_step_args b = *a;
+    b.two_step = 0;
+    const int rc = sizeof(S) == 4 ? step_fused_f32(h, &b, st) : step_fused_f64(h, &b, st);
+    a->result_swapped = b.result_swapped;
+    return rc;
   }
   wf::T2Aux x{};
   t2_aux(sh, g, a, x);
