@@ -496,12 +496,17 @@ int wf_wake_wp(const void *capture, int32_t dtype, int32_t nlines, int64_t cap_s
   if (dtype != WF_F64 && dtype != WF_F32) return fail(WF_EINVAL, "wf_wake_wp: bad dtype");
   if (ns == 0) return WF_OK;
   hipStream_t st = (hipStream_t)stream;
-  const size_t lds = nz <= wf::WP_COLS_MAX ? (size_t)nz * wf::WP_NS * sizeof(int) : 0;
+  int dev = 0, ncu = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return fail(WF_EHIP, "wf_wake_wp: device attributes");
+  const bool kept = wf::wp_keep_columns(nlines, nz, ns, nt, ncu);
+  const size_t lds = kept ? (size_t)nz * wf::WP_NS * sizeof(int) : 0;
 #define WF_WP_LAUNCH(S, CM)                                                                   \
   hipLaunchKernelGGL((wf::k_wake_wp<S, CM>), dim3(nblocks(ns, wf::WP_NS)),                    \
                      dim3(wf::WP_THREADS), lds, st,                                           \
                      (const S *)capture, nlines, cap_samples, Nz, k0, nz, z, dz, s, ns, v,    \
-                     zref_v, t0, ti, dt, nt, ncols, qe12, WP3d)
+                     zref_v, t0, ti, dt, nt, ncols, qe12, kept, WP3d)
   if (dtype == WF_F64) {
     if (counter_moving) WF_WP_LAUNCH(double, true);
     else WF_WP_LAUNCH(double, false);

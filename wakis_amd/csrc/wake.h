@@ -26,23 +26,33 @@ namespace wf {
 // samples per workgroup spread the gather over the CUs (the lane-per-sample
 // form had 1 to 30 workgroups, each waiting for its loads row by row). The
 // columns hold for every line and are formed once (two FP64 divisions each)
-// where they fit in LDS. us, lane per sample -> this: 9 lines of 128 rows, 2,062
+// where LDS has room for them (wp_keep_columns). us, lane per sample -> this: 9 lines of 128 rows, 2,062
 // samples, FP64 443 -> 39; 9 x 300 rows, 8,000 samples, FP64 1,115 -> 94; 9 x 462
 // rows, 3,622 samples, FP32 2,506 -> 174.
 constexpr int WP_NS = 16, WP_KC = 128, WP_THREADS = 320;
-// rows of columns kept in LDS beside the two product buffers
+// rows of columns that LDS holds beside the two product buffers
 constexpr int WP_COLS_MAX = 1800;
+// Whether a launch keeps them: for several lines, and unless they hold a CU to one
+// workgroup (past 768 rows) where the launch has more. us, kept / formed on each
+// line, FP64, dz = 1.75 v dt: 9 lines of 1,000 rows, 2,000 samples 296 / 464, 20,000
+// 1,841 / 1,128, 130,000 11,674 / 6,026; of 300 rows, 20,000 264 / 345; one line of
+// 500 rows, 130,000 samples 585 / 360, of 1,000 rows 1,730 / 686.
+inline bool wp_keep_columns(int nlines, int nz, int64_t ns, int64_t nt, int ncu) {
+  constexpr int64_t LDS_CU = 163840, prod = 2 * WP_KC * WP_NS * (int64_t)sizeof(double);
+  if (nlines < 2 || nz > WP_COLS_MAX || nt >= (int64_t)1 << 31) return false;
+  const int64_t per_cu = LDS_CU / (prod + (int64_t)nz * WP_NS * (int64_t)sizeof(int));
+  return per_cu > 1 || (ns + WP_NS - 1) / WP_NS <= ncu;
+}
 
 template <typename S, bool CM>
 __global__ void __launch_bounds__(WP_THREADS)
 k_wake_wp(const S *__restrict__ cap, int nlines, int64_t cap_samples, int Nz, int k0, int nz,
           const double *__restrict__ z, const double *__restrict__ dz,
           const double *__restrict__ s, int64_t ns, double v, double zref_v, double t0,
-          double ti, double dt, int64_t nt, int64_t ncols, double qe12,
+          double ti, double dt, int64_t nt, int64_t ncols, double qe12, bool kept,
           double *__restrict__ WP3d) {
   __shared__ double prod[2][WP_KC * WP_NS];
-  extern __shared__ int wp_cols[];  // [nz][WP_NS], or none
-  const bool kept = nz <= WP_COLS_MAX && nt < (int64_t)1 << 31;
+  extern __shared__ int wp_cols[];  // [nz][WP_NS] if kept
   const int sub = (int)threadIdx.x & (WP_NS - 1);
   const int64_t n = (int64_t)blockIdx.x * WP_NS + sub;
   const double sn = s[n < ns ? n : ns - 1];
