@@ -792,10 +792,9 @@ class SolverFIT3D(RoutinesMixin):
             args.code_escape = int(self._code_escape)
             # weight codes where pairs of steps run: built by the first longer call
             # (100 to 200 us, a few steps' gain at any size), then kept
-            if (self.use_weight_codes and self.dtype == np.float32
-                    and self._pairs_apply(args, prepared=True)
+            if (self.use_weight_codes and args.beam_table and self.dtype == np.float32
                     and (args.nsteps >= 64 or self._wkey == (self._lut_key, float(self.dt)))
-                    and self._weight_table()):
+                    and self._pairs_apply(args, prepared=True) and self._weight_table()):
                 args.wcode, args.wtab = _lib.ptr(self._wcode), _lib.ptr(self._wtab)
                 args.nw = self._wtab.shape[0]
         if args.jmode == _lib.WF_J_FULL and not args.conductive:
@@ -873,12 +872,15 @@ class SolverFIT3D(RoutinesMixin):
         arguments have been through ``_prepare_fused``."""
         if not prepared and not self._prepare_fused(args):
             return False
-        size = np.dtype(self.dtype).itemsize
-        box = all(h > l for l, h in zip(args.box_lo, args.box_hi))
-        return bool(args.two_step and args.code and args.zero_masked and not args.code_escape
-                    and args.beam_table and self._pairs_in_reach() and args.variant == 0
-                    and args.full_rows <= 0 and args.cells_per_lane in (0, 16 // size)
-                    and not box and not args.traj_E and (not args.mon_acc or args.mon_work))
+        if not (args.beam_table and args.two_step and args.code and args.zero_masked
+                and not args.code_escape and args.variant == 0 and args.full_rows <= 0
+                and not args.traj_E and (not args.mon_acc or args.mon_work)):
+            return False
+        lo, hi = args.box_lo, args.box_hi
+        return ((args.cells_per_lane == 0
+                 or args.cells_per_lane == 16 // np.dtype(self.dtype).itemsize)
+                and not (hi[0] > lo[0] and hi[1] > lo[1] and hi[2] > lo[2])
+                and self._pairs_in_reach())
 
     def _pairs_in_reach(self):
         """Whether the two-step kernel's 32-bit offsets reach every array (t2_limits.h)."""
