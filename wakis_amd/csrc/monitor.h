@@ -36,7 +36,7 @@ k_monitor(const S *__restrict__ E, int64_t N, const P *__restrict__ phase, int n
 // The same for the E of nk <= MON_STEPS steps in turn: each accumulator crosses
 // memory once for all of them (16 bytes read and written per component,
 // frequency and cell, against 4 or 8 for a step's E), the sum in the same order.
-// Bound by those bytes: 96x96x160 FP32, 2 frequencies, 57 us for 8 steps at 7.4 TB/s
+// Bound by those bytes: 96x96x160 FP32, 2 frequencies, 59 us for 8 steps at 7.2 TB/s
 // (the accumulators stay in the last cache), 46 us for one step before.
 constexpr int MON_STEPS = 8;
 template <typename S>

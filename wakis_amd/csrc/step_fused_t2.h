@@ -52,9 +52,9 @@
 //
 // What bounds it: memory on large FP32 grids (256x256x512: 1.70 GB per launch at
 // 5.1 TB/s, the rate of a device copy); elsewhere the chain of a plane, LDS passes
-// and the instructions its 12 waves issue between two barriers (663 a plane on
-// weight codes, 408 of them the arithmetic of the exact row sums; 1,110 on material
-// codes). One branch per update and none per cell, buffer loads that return zeros
+// and the instructions its 12 waves issue between two barriers (a wave and plane, by
+// the counters at 256x256x512: 383 VALU and 79 LDS on weight codes, 555 and 94 on
+// material codes). One branch per update and none per cell, buffer loads that return zeros
 // off the grid, own neighbours from registers. us per step, one step per launch (or
 // rows of one wave and a branch per cell, *) -> this form on material codes -> now:
 // 256x256x512 FP32 197* -> 188 -> 165, 200x200x400 FP32 with conduction 149* -> 111
@@ -81,7 +81,8 @@ struct T2Aux {
 };
 
 // Threads of a workgroup at most, and LDS slots per block of the staged E0, H1,
-// E1, H2 (a buffer of R rows takes R * QS + 1 slots): 144.4 KB of the CU's 160
+// E1, H2 (a buffer of R rows takes R * QS + 1 slots): 126.7 KB FP32, 132.6 KB FP64
+// of the CU's 160
 constexpr int T2_NT = 768;
 struct T2Slots {
   static constexpr int E0 = 832, H1 = 768, E1 = 704, H2 = 704;
